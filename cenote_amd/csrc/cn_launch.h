@@ -79,7 +79,7 @@ hipError_t launch_raygen(hipStream_t stream, uint32_t* counters, uint32_t counte
 hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const SceneView& s, const PathPool& p,
                          const WaveTargets& tg, uint32_t* counters, const JobRecord* jobs, uint32_t job_count,
                          uint32_t base, uint32_t range_count, uint32_t bounce, uint32_t light_sampling, int counting,
-                         bool tail, uint32_t* tail_claims, uint32_t compute_units, Profiler* prof);
+                         bool tail, uint32_t max_bounces, uint32_t compute_units, Profiler* prof);
 
 // Fold every job's slots into its film sums (jobs sorted by pixel base;
 // total_pixels is the sum of the jobs' view pixels).

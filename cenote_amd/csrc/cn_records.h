@@ -35,14 +35,18 @@ constexpr uint32_t COUNTER_STRIDE = 32;   // u32 words per counter: one 128-byte
 // Most pixel ranges a single wave may walk (pixels / capacity, rounded up).
 constexpr uint32_t MAX_RANGES = 64;
 // Counters one range holds: Q_COUNT x QUEUE_SPLIT per bounce, plus one
-// spare bounce, then QUEUE_SPLIT striped item counters for the tail launch.
+// spare bounce, then QUEUE_SPLIT striped item counters for the tail launch,
+// then as many striped chunk counters for each bounce's trace launch.
 constexpr uint32_t counter_lines_per_range(uint32_t max_bounces) {
-    return (max_bounces + 1) * Q_COUNT * QUEUE_SPLIT + QUEUE_SPLIT;
+    return (max_bounces + 1) * Q_COUNT * QUEUE_SPLIT + QUEUE_SPLIT + max_bounces * QUEUE_SPLIT;
 }
 // The first of the tail launch's striped item counters (the others follow,
-// COUNTER_STRIDE words apart).
+// COUNTER_STRIDE words apart), and of bounce b's trace launch.
 constexpr uint32_t tail_claim_index(uint32_t max_bounces) {
     return (max_bounces + 1) * Q_COUNT * QUEUE_SPLIT * COUNTER_STRIDE;
+}
+constexpr uint32_t trace_claim_index(uint32_t max_bounces, uint32_t bounce) {
+    return tail_claim_index(max_bounces) + (1 + bounce) * QUEUE_SPLIT * COUNTER_STRIDE;
 }
 constexpr uint32_t counters_per_range(uint32_t max_bounces) {
     return counter_lines_per_range(max_bounces) * COUNTER_STRIDE;

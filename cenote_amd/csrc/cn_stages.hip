@@ -18,6 +18,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "cn_launch.h"
 #include "cn_math.h"
 #include "cn_records.h"
@@ -244,68 +246,43 @@ __global__ __launch_bounds__(BLOCK) void k_shade_miss(SceneView s, PathPool p, W
 // bounce's trace_shadow (trace_shadow.slang:27-72) ------------------------------
 //
 // Bounce b's extension rays and bounce b-1's shadow rays are independent, so
-// one launch walks both: items [0, n_ray) are rays, [n_ray, n_ray + n_shadow)
-// are shadow records. The reference's pass order is kept where it shows:
-// a slot's shadow add from bounce b-1 lands before bounce b's shading adds.
-// Two half-empty launches per bounce become one fuller one, which is what
-// the deep, sparse bounces need.
+// one launch walks both queues. The reference's pass order is kept where it
+// shows: a slot's shadow add from bounce b-1 lands before bounce b's shading
+// adds. Two half-empty launches per bounce become one fuller one, which is
+// what the deep, sparse bounces need.
 
 // The 8-wide walk holds eight keys and refs through its sorting network:
 // at eight waves per SIMD (64 VGPRs) it spills, so it runs at fewer.
 #ifndef TRACE8_WAVES
 #define TRACE8_WAVES 7
 #endif
+constexpr uint32_t TRACE4_WAVES = 8;
 // The tail kernel holds shading's registers and a traversal: three waves
 // per SIMD, as shade_surface.
 #ifndef TAIL_WAVES
 #define TAIL_WAVES 3
 #endif
 
-// COUNT: accumulate node and triangle fetches (the counting pass); the
-// timed form keeps no counters. Eight waves per SIMD (64 VGPRs; LDS 8 x 16
-// KB per CU) fit without scratch: traversal waits on memory, so every
-// extra wave hides latency.
-// CAMERA: the bounce-0 form, which also shades the camera rays that escape
-// (a separate instantiation, so the later bounces' kernel keeps its
-// registers).
-template <bool COUNT, bool W8, bool CAMERA>
-__global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu(W8 ? TRACE8_WAVES : 8))) void k_trace(SceneView s, PathPool p, WaveTargets tg, uint32_t* counters,
-                                                           const JobRecord* __restrict__ jobs, uint32_t job_count,
-                                                           uint32_t base, uint32_t range_count, uint32_t bounce,
-                                                           uint32_t light_sampling) {
+// Bounce 0: the camera rays of a range, generated here, and their misses
+// shaded in place. COUNT: accumulate node and triangle fetches (the counting
+// pass); the timed form keeps no counters.
+template <bool COUNT, bool W8>
+__global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu(W8 ? TRACE8_WAVES : 8))) void k_trace_camera(
+    SceneView s, PathPool p, WaveTargets tg, uint32_t* counters, const JobRecord* __restrict__ jobs, uint32_t job_count,
+    uint32_t base, uint32_t n, uint32_t light_sampling) {
     __shared__ uint32_t lds_stack[STACK_LDS * TRAVERSAL_BLOCK];
-    // Bounce 0 traces the camera paths: item i is path i.
-    const uint32_t n_ray = CAMERA ? range_count : queue_total(counters, bounce, Q_RAY);
-    const uint32_t n = n_ray + (CAMERA ? 0u : queue_total(counters, bounce - 1, Q_SHADOW));
-    const uint32_t* rays = p.ray_queue[bounce & 1];
     const uint32_t lanes = gridDim.x * TRAVERSAL_BLOCK;
     Stack st = make_stack(lds_stack, p.stack_overflow, lanes, blockIdx.x * TRAVERSAL_BLOCK + threadIdx.x);
-    const uint32_t mask = CAMERA ? MASK_CAMERA : MASK_ALL;
-    uint32_t ray_nodes = 0, ray_tris = 0, shadow_nodes = 0, shadow_tris = 0;
+    uint32_t ray_nodes = 0, ray_tris = 0;
     for (uint32_t first = blockIdx.x * TRAVERSAL_BLOCK; first < n; first += lanes) {
-        const uint32_t i = first + threadIdx.x;
-        const bool is_ray = i < n_ray;
-        uint32_t path = 0, cls = 0;
+        const uint32_t path = first + threadIdx.x;  // item i is path i, the camera path of slot base + i
+        const bool is_ray = path < n;
+        uint32_t cls = 0;
         bool hit = false;
         if (is_ray) {
-            v3 o, d;
-            uint2 key;
-            CameraPath cam;
-            if constexpr (CAMERA) {
-                // bounce 0 generates the camera path of slot base + i
-                path = i;
-                cam = camera_path(jobs, job_count, base + i);
-                o = cam.o;
-                d = cam.d;
-                key = cam.key;
-            } else {
-                path = rays[queue_slot(counters, bounce, Q_RAY, i, p.sub_capacity)];
-                o = xyz(p.origin[path]);
-                d = xyz(p.direction[path]);
-                key = p.key[path];
-            }
+            const CameraPath cam = camera_path(jobs, job_count, base + path);
             TraceHit h;
-            if constexpr (CAMERA && !W8 && !COUNT) {
+            if constexpr (!W8 && !COUNT) {
                 // Camera rays walk the 4-wide tree as a wave (trace_packet),
                 // on the wave's own rows of the stack array. The counting
                 // form keeps the per-ray walk, whose fetches the byte model
@@ -313,51 +290,206 @@ __global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu
                 static_assert(TRAVERSAL_BLOCK / 64 * PACKET_STACK_ROW <= STACK_LDS * TRAVERSAL_BLOCK,
                               "the packet stack rows fit the block's LDS stack");
                 lds_u32* wstack = (lds_u32*)lds_stack + (threadIdx.x / 64) * PACKET_STACK_ROW;
-                h = trace_packet(s, o, d, mask, key.x, key.y, wstack, ray_nodes, ray_tris);
+                h = trace_packet(s, cam.o, cam.d, MASK_CAMERA, cam.key.x, cam.key.y, wstack, ray_nodes, ray_tris);
             } else {
-                h = trace_closest<W8>(s, o, d, 1e30f, mask, st, key.x, key.y, bounce, ray_nodes, ray_tris);
+                h = trace_closest<W8>(s, cam.o, cam.d, 1e30f, MASK_CAMERA, st, cam.key.x, cam.key.y, 0, ray_nodes,
+                                      ray_tris);
             }
-            hit = h.hit;
+            hit = h.hit();
             if (hit) {
+                // the path's records, for its shading and later bounces
                 p.hit[path] = make_uint4(h.inst, h.prim, __float_as_uint(h.b1), __float_as_uint(h.b2));
-                if constexpr (CAMERA) {
-                    // the path's records, for its shading and later bounces
-                    p.origin[path] = F4(o, __uint_as_float(cam.max_bounces));  // w: the path's depth cap
-                    p.direction[path] = F4(d, cam.cos_forward);
-                    p.key[path] = key;
-                }
-            } else if constexpr (CAMERA) {
+                p.origin[path] = F4(cam.o, __uint_as_float(cam.max_bounces));  // w: the path's depth cap
+                p.direction[path] = F4(cam.d, cam.cos_forward);
+                p.key[path] = cam.key;
+            } else {
                 // A camera ray that escapes is shaded here: no other item of
                 // this launch adds to its slot (bounce 0 carries no
                 // connections). A camera path's throughput, (1, 1, 1) with no
                 // previous pdf, is never stored.
-                miss_shade(s, tg, base + path, d, camera_throughput(), 0, light_sampling);
+                miss_shade(s, tg, base + path, cam.d, camera_throughput(), 0, light_sampling);
             }
             cls = (h.flags >> TRI_CLASS_SHIFT) & (MATERIAL_CLASSES - 1);
-        } else if (i < n) {
-            const uint32_t j = queue_slot(counters, bounce - 1, Q_SHADOW, i - n_ray, p.sub_capacity);
-            const float4 o4 = p.shadow_origin[j];
-            const float4 d4 = p.shadow_dir[j];
-            const float4 c4 = p.shadow_contrib[j];
-            const uint32_t target = __float_as_uint(c4.w);
-            // Any solid non-target hit short of the light's own distance
-            // (tmax / 1.001 for a triangle target) lies in front of the
-            // target, so it occludes without finding the closest hit.
-            const float t_early = target == LIGHT_NONE ? 3.0e38f : o4.w * 0.998f;
-            const float att = trace_visibility<W8>(s, xyz(o4), xyz(d4), o4.w, target, p.shadow_prim[j], t_early, st,
-                                               shadow_nodes, shadow_tris);
-            if (att > 0.0f) add_pixel(tg.radiance, __float_as_uint(d4.w), xyz(c4) * att, 0.0f);
         }
-        if (first < n_ray) {  // uniform per block: some wave of this block holds rays
-            const uint32_t split = chunk_split(first);
-            const uint32_t hs = wave_claim(&counters[counter_index(bounce, Q_HIT, split)], is_ray && hit);
-            const uint32_t ms = wave_claim(&counters[counter_index(bounce, Q_MISS, split)], is_ray && !hit);
-            if (is_ray) {
+        const uint32_t split = chunk_split(first);
+        const uint32_t hs = wave_claim(&counters[counter_index(0, Q_HIT, split)], is_ray && hit);
+        wave_claim(&counters[counter_index(0, Q_MISS, split)], is_ray && !hit);  // counted, and shaded above
+        if (hit) p.hit_queue[split * p.sub_capacity + hs] = path | (cls << HIT_PATH_BITS);
+    }
+    if constexpr (COUNT) {
+        wave_add_u64(&p.traversal_counts[0], ray_nodes);
+        wave_add_u64(&p.traversal_counts[1], ray_tris);
+    }
+}
+
+// Later bounces. The launch is one grid the chip holds at once; its waves
+// take the queues in chunks of consecutive entries, the first by wave number
+// and further ones as they finish (one atomic on one of QUEUE_SPLIT striped
+// counters), and a wave walks a chunk with its lanes refilled and its steps
+// chosen by vote (walk_many). What a chunk's rays hit is kept as a byte per
+// ray in LDS and pushed to the hit and miss queues in the chunk's order once
+// all are done, so the queues' order, and with it the locality of the shading
+// kernels, is that of a walk without refilling.
+//
+// What bounds it: VALU issue and the vector memory pipe alike (the first
+// bounce of the 2M-triangle scene seen from inside: VALU issue above 0.9 of
+// the mix's rate, the data return unit busy 0.95 of the time, 0.28 of the
+// lanes active when every lane kept its ray until its wave was done). Refilled
+// and voted, that launch (29M rays and 6M connections) went from 14.1 to 9.3
+// ms; the frame's trace time from 32.8 to 26.2 ms there, 13.6 to 11.7 on the
+// outside view, 10.7 to 8.1 on the chart. Eight waves per SIMD (64 VGPRs; LDS
+// 8 x 18 KB per CU) measured 25.8 ms against 26.0 at seven and at six.
+// Chunks: 256 to 1,024 entries within 2% (512 kept); a fixed share per wave
+// instead of claims 27.8 ms. The grid of 16,384 blocks that this replaces took
+// 80 us to dispatch even for a few hundred rays; a launch of 800 rays now
+// takes 46 us, their longest chain of fetches.
+constexpr uint32_t TRACE_CHUNK_MAX = 512;
+constexpr uint32_t TRACE_CHUNK_MIN = 4;
+
+template <bool COUNT, bool W8>
+__global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu(W8 ? TRACE8_WAVES : TRACE4_WAVES))) void k_trace(
+    SceneView s, PathPool p, WaveTargets tg, uint32_t* counters, uint32_t* claims, uint32_t bounce) {
+    __shared__ uint32_t lds_stack[STACK_LDS * TRAVERSAL_BLOCK];
+    __shared__ uint8_t lds_marks[TRAVERSAL_BLOCK / 64][TRACE_CHUNK_MAX];
+    constexpr uint32_t BLOCK_WAVES = TRAVERSAL_BLOCK / 64;
+    const uint32_t n_ray = queue_total(counters, bounce, Q_RAY);
+    const uint32_t n_shadow = queue_total(counters, bounce - 1, Q_SHADOW);
+    const uint32_t lane = __lane_id();
+    const uint32_t waves = gridDim.x * BLOCK_WAVES;
+    const uint32_t wave = wave_uniform(blockIdx.x * BLOCK_WAVES + threadIdx.x / 64);
+    // A chunk per wave of the grid where TRACE_CHUNK_MAX entries each suffice:
+    // a multiple of 64, or a power of two from TRACE_CHUNK_MIN below that (a
+    // small launch lasts as long as its longest wave, whose turns wait on the
+    // fetches of all its rays one after another, so few rays go over many
+    // waves: the 720p chart's sparse bounces 45 to 58 us against 63 to 75 with
+    // chunks of 64 at least; 1, 4 and 16 at least measured within 3%).
+    const uint32_t share = (n_ray + n_shadow + waves - 1) / waves;
+    uint32_t size = TRACE_CHUNK_MIN;
+    if (share <= 64)
+        while (size < share) size *= 2;
+    else
+        size = min((share + 63) / 64 * 64, TRACE_CHUNK_MAX);
+    const uint32_t ray_chunks = (n_ray + size - 1) / size;
+    const uint32_t chunks = ray_chunks + (n_shadow + size - 1) / size;
+    if (wave >= chunks) return;
+    const uint32_t* rays = p.ray_queue[bounce & 1];
+    Stack st = make_stack(lds_stack, p.stack_overflow, gridDim.x * TRAVERSAL_BLOCK,
+                          blockIdx.x * TRAVERSAL_BLOCK + threadIdx.x);
+    uint8_t* marks = lds_marks[threadIdx.x / 64];
+    uint32_t ray_nodes = 0, ray_tris = 0, shadow_nodes = 0, shadow_tris = 0;
+    uint32_t stripe = wave % QUEUE_SPLIT;
+    uint32_t chunk = wave;
+    while (true) {
+        Ray r{};
+        TraceHit best{};
+        if (chunk < ray_chunks) {
+            const uint32_t first = chunk * size, count = min(size, n_ray - first);
+            uint32_t path = 0, item = 0;
+            walk_many(
+                tree_of<W8>(s), s.tris, r, best.t, st, count, ray_nodes, ray_tris,
+                [&](uint32_t i) {
+                    item = i;
+                    path = rays[queue_slot(counters, bounce, Q_RAY, first + i, p.sub_capacity)];
+                    const v3 o = xyz(p.origin[path]), d = xyz(p.direction[path]);
+                    r = make_ray(o, d);
+                    best = no_hit(1e30f);
+                },
+                [&](const BvhTriangle& tri) {
+                    closest_triangle(s, tri, r, MASK_ALL, [&] { return p.key[path]; }, bounce, best);
+                    return false;
+                },
+                [&] {
+                    if (best.hit())
+                        p.hit[path] =
+                            make_uint4(best.inst, best.prim, __float_as_uint(best.b1), __float_as_uint(best.b2));
+                    const uint32_t cls = (best.flags >> TRI_CLASS_SHIFT) & (MATERIAL_CLASSES - 1);
+                    marks[item] = uint8_t(best.hit() ? 1u + cls : 0u);
+                });
+            // The wave's own marks: written and read by this wave alone.
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            for (uint32_t k = 0; k < count; k += 64) {
+                const uint32_t split = (first + k) / QUEUE_CHUNK % QUEUE_SPLIT;
                 const uint32_t at = split * p.sub_capacity;
-                if (hit) p.hit_queue[at + hs] = path | (cls << HIT_PATH_BITS);
-                else if (!CAMERA) p.miss_queue[at + ms] = path;  // bounce 0's are counted, and shaded above
+                const bool valid = k + lane < count;
+                const uint32_t mark = valid ? marks[k + lane] : 0u;
+                const uint32_t entry =
+                    valid ? rays[queue_slot(counters, bounce, Q_RAY, first + k + lane, p.sub_capacity)] : 0u;
+                const bool hit = mark != 0;
+                const uint32_t hs = wave_claim(&counters[counter_index(bounce, Q_HIT, split)], hit);
+                const uint32_t ms = wave_claim(&counters[counter_index(bounce, Q_MISS, split)], valid && !hit);
+                if (hit) p.hit_queue[at + hs] = entry | ((mark - 1u) << HIT_PATH_BITS);
+                else if (valid) p.miss_queue[at + ms] = entry;
             }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        } else {
+            const uint32_t first = (chunk - ray_chunks) * size, count = min(size, n_shadow - first);
+            uint32_t record = 0, item = 0, target = 0, target_prim = 0;
+            float t_early = 0.0f;
+            constexpr uint32_t OCCLUDED = 1u, TRANSLUCENT = 2u;
+            uint32_t state = 0;
+            walk_many(
+                tree_of<W8>(s), s.tris, r, best.t, st, count, shadow_nodes, shadow_tris,
+                [&](uint32_t i) {
+                    item = i;
+                    record = queue_slot(counters, bounce - 1, Q_SHADOW, first + i, p.sub_capacity);
+                    const float4 o4 = p.shadow_origin[record];
+                    const v3 d = xyz(p.shadow_dir[record]);
+                    target = __float_as_uint(p.shadow_contrib[record].w);
+                    target_prim = p.shadow_prim[record];
+                    t_early = early_occlusion(target, o4.w);
+                    r = make_ray(xyz(o4), d);
+                    best = no_hit(o4.w);
+                    state = 0;
+                },
+                [&](const BvhTriangle& tri) {
+                    bool translucent = false;
+                    const bool occluded = visibility_triangle(tri, r, target, target_prim, t_early, best, translucent);
+                    state |= (occluded ? OCCLUDED : 0u) | (translucent ? TRANSLUCENT : 0u);
+                    return occluded;
+                },
+                [&] {
+                    const bool visible =
+                        !(state & OCCLUDED) && (!best.hit() || (best.inst == target && best.prim == target_prim));
+                    const bool attenuated = visible && (state & TRANSLUCENT);
+                    marks[item] = attenuated ? 1u : 0u;
+                    if (attenuated) p.shadow_origin[record].w = best.t;  // where the attenuating walk ends
+                    if (visible && !attenuated)
+                        add_pixel(tg.radiance, __float_as_uint(p.shadow_dir[record].w), xyz(p.shadow_contrib[record]),
+                                  0.0f);
+                });
+            // The rare connections that are visible through fractional
+            // opacity: one more walk each.
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            for (uint32_t k = lane; k < count; k += 64) {
+                if (!marks[k]) continue;
+                const uint32_t j = queue_slot(counters, bounce - 1, Q_SHADOW, first + k, p.sub_capacity);
+                const float4 o4 = p.shadow_origin[j], d4 = p.shadow_dir[j], c4 = p.shadow_contrib[j];
+                const float att = shadow_attenuation<W8>(s, make_ray(xyz(o4), xyz(d4)), o4.w, __float_as_uint(c4.w),
+                                                         p.shadow_prim[j], st, shadow_nodes);
+                if (att > 0.0f) add_pixel(tg.radiance, __float_as_uint(d4.w), xyz(c4) * att, 0.0f);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
+        // The next chunk: those past the first `waves` are dealt by the
+        // striped counters, stripe k dealing waves + k, waves + k +
+        // QUEUE_SPLIT, ... A spent stripe sends the wave to one that a single
+        // read of all shows open (counters only grow, so when none is open
+        // none will be).
+        if (chunks <= waves) break;
+        while (true) {
+            uint32_t c = 0;
+            if (lane == 0) c = atomicAdd(&claims[stripe * COUNTER_STRIDE], 1u);
+            c = wave_uniform(c);
+            chunk = waves + stripe + QUEUE_SPLIT * c;
+            if (chunk < chunks) break;
+            uint32_t taken = 0;
+            if (lane < QUEUE_SPLIT)
+                taken = __hip_atomic_load(&claims[lane * COUNTER_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t open = __ballot(lane < QUEUE_SPLIT && waves + lane + QUEUE_SPLIT * taken < chunks);
+            if (open == 0) break;
+            stripe = __ffsll((unsigned long long)open) - 1;
+        }
+        if (chunk >= chunks) break;
     }
     if constexpr (COUNT) {
         unsigned long long* c = p.traversal_counts + 4 * bounce;  // this launch's bounce row
@@ -870,42 +1002,36 @@ __global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu
                 // The owner walks the next ray, the mate the connection.
                 v3 o = sh.origin, d = sh.direction;
                 float tmax = sh.tmax;
-                uint2 key = make_uint2(0u, 0u);
                 if (!helper && next) {
                     o = xyz(p.origin[path]);
                     d = xyz(p.direction[path]);
-                    key = p.key[path];
                 }
                 if (!helper) tmax = 1e30f;
-                const SlabRay r = make_slab(o, d);
-                const WRay w = make_wray(o, d);
-                TraceHit best{false, tmax, 0u, 0u, 0.0f, 0.0f, 0u};
+                const Ray r = make_ray(o, d);
+                TraceHit best = no_hit(tmax);
                 bool occluded = false, translucent = false;
-                // As the trace kernel takes a connection: a solid hit short of a
-                // triangle light occludes without the closest hit.
-                const float t_early = sh.instance == LIGHT_NONE ? 3.0e38f : sh.tmax * 0.998f;
+                const float t_early = early_occlusion(sh.instance, sh.tmax);
                 if (helper ? connect : next) {
                     walk(tree_of<W8>(s), r, best.t, st, nodes, [&](uint32_t ref) {
                         if (helper) {
-                            occluded = visibility_leaf(s, w, ref, sh.instance, sh.primitive, t_early, best, translucent,
+                            occluded = visibility_leaf(s, r, ref, sh.instance, sh.primitive, t_early, best, translucent,
                                                        tris);
                             return occluded;
                         }
-                        closest_leaf(s, TrisPerLane{s.tris}, w, ref, MASK_ALL, key.x, key.y, b + 1, best, tris);
+                        closest_leaf(s, TrisPerLane{s.tris}, r, ref, MASK_ALL, [&] { return p.key[path]; }, b + 1, best, tris);
                         return false;
                     });
                 }
                 float att = 0.0f;
-                if (helper && connect && !occluded && !(best.hit && !(best.inst == sh.instance && best.prim == sh.primitive)))
-                    att = translucent ? shadow_attenuation<W8>(s, r, w, best.hit ? best.t : sh.tmax, sh.instance,
-                                                               sh.primitive, st, nodes)
+                if (helper && connect && !occluded && !(best.hit() && !(best.inst == sh.instance && best.prim == sh.primitive)))
+                    att = translucent ? shadow_attenuation<W8>(s, r, best.t, sh.instance, sh.primitive, st, nodes)
                                       : 1.0f;
                 att = __shfl(att, mate);
                 if (!helper && connect && att > 0.0f) add_pixel(tg.radiance, sh.pixel, sh.contrib * att, 0.0f);
             if (!next) {
                 live = false;
             } else {
-                const bool hit = __shfl(best.hit ? 1 : 0, owner) != 0;
+                const bool hit = __shfl(best.hit() ? 1 : 0, owner) != 0;
                 if (!hit) {
                     if (!helper) miss_path(s, p, tg, path, base, b + 1, light_sampling);
                     live = false;
@@ -1169,10 +1295,10 @@ __global__ __launch_bounds__(TRAVERSAL_BLOCK) void k_first_hits(SceneView s, Cam
         float cf;
         camera_ray(cam, width, height, pixel, sample, &o, &d, &cf);
         const TraceHit h = trace_closest<W8>(s, o, d, 1e30f, MASK_CAMERA, st, pixel, sample, 0, nodes, tris);
-        inst_out[pixel] = h.hit ? h.inst : 0xffffffffu;
-        prim_out[pixel] = h.hit ? h.prim : 0xffffffffu;
-        bary_out[2 * pixel] = h.hit ? h.b1 : 0.0f;
-        bary_out[2 * pixel + 1] = h.hit ? h.b2 : 0.0f;
+        inst_out[pixel] = h.hit() ? h.inst : 0xffffffffu;
+        prim_out[pixel] = h.hit() ? h.prim : 0xffffffffu;
+        bary_out[2 * pixel] = h.hit() ? h.b1 : 0.0f;
+        bary_out[2 * pixel + 1] = h.hit() ? h.b2 : 0.0f;
     }
 }
 
@@ -1225,28 +1351,44 @@ hipError_t launch_raygen(hipStream_t stream, uint32_t* counters, uint32_t counte
 hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const SceneView& s, const PathPool& p,
                          const WaveTargets& tg, uint32_t* counters, const JobRecord* jobs, uint32_t job_count,
                          uint32_t base, uint32_t range_count, uint32_t bounce, uint32_t light_sampling, int counting,
-                         bool tail, uint32_t* tail_claims, uint32_t compute_units, Profiler* prof) {
-    const uint32_t trace_grid = shape.trace_blocks;
+                         bool tail, uint32_t max_bounces, uint32_t compute_units, Profiler* prof) {
     const uint32_t light_grid = grid_for(range_count, shape.light_blocks);
     // Bounce b's rays and bounce b-1's shadow rays share one launch; the
     // last bounce shades terminally and leaves no shadow rays behind.
     if (prof) prof->begin(K_TRACE);
     const bool wide = shape.bvh_width == 8 && s.nodes8 != nullptr;
-#define CN_TRACE(COUNT, W8, CAMERA)                                                                                 \
-    hipLaunchKernelGGL((k_trace<COUNT, W8, CAMERA>), dim3(trace_grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg,   \
-                       counters, jobs, job_count, base, range_count, bounce, light_sampling)
-#define CN_TRACE_CAMERA(COUNT, W8)   \
-    if (bounce == 0) CN_TRACE(COUNT, W8, true); \
-    else CN_TRACE(COUNT, W8, false)
-    if (counting) {
-        if (wide) CN_TRACE_CAMERA(true, true);
-        else CN_TRACE_CAMERA(true, false);
-    } else {
-        if (wide) CN_TRACE_CAMERA(false, true);
-        else CN_TRACE_CAMERA(false, false);
-    }
-#undef CN_TRACE_CAMERA
+    if (bounce == 0) {
+        const uint32_t grid = grid_for(range_count, shape.trace_blocks);
+#define CN_TRACE(COUNT, W8)                                                                                     \
+    hipLaunchKernelGGL((k_trace_camera<COUNT, W8>), dim3(grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg, counters, \
+                       jobs, job_count, base, range_count, light_sampling)
+        if (counting) {
+            if (wide) CN_TRACE(true, true);
+            else CN_TRACE(true, false);
+        } else {
+            if (wide) CN_TRACE(false, true);
+            else CN_TRACE(false, false);
+        }
 #undef CN_TRACE
+    } else {
+        // One grid the chip holds at once, and no more blocks than hold the
+        // most rays and connections the range can send (one of each per path).
+        const uint32_t waves_per_simd = wide ? TRACE8_WAVES : TRACE4_WAVES;
+        const uint32_t resident = std::min(shape.trace_blocks, (compute_units ? compute_units : 1u) * waves_per_simd);
+        const uint32_t grid = uint32_t(std::min<uint64_t>(resident, (2ull * range_count + BLOCK - 1) / BLOCK));
+        uint32_t* claims = counters + trace_claim_index(max_bounces, bounce);
+#define CN_TRACE(COUNT, W8)                                                                                            \
+    hipLaunchKernelGGL((k_trace<COUNT, W8>), dim3(grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg, counters, claims, \
+                       bounce)
+        if (counting) {
+            if (wide) CN_TRACE(true, true);
+            else CN_TRACE(true, false);
+        } else {
+            if (wide) CN_TRACE(false, true);
+            else CN_TRACE(false, false);
+        }
+#undef CN_TRACE
+    }
     if (prof) prof->end(K_TRACE);
     if (tail) {
         // The waves the chip holds at once (TAIL_WAVES per SIMD: one
@@ -1254,14 +1396,14 @@ hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const Sce
         // lanes the traversal stack's spill area is sized for): the pairs
         // claim items until none are left.
         const uint32_t resident = (compute_units ? compute_units : 1u) * TAIL_WAVES;
-        const uint32_t tail_grid = resident < trace_grid ? resident : trace_grid;
+        const uint32_t tail_grid = std::min(resident, shape.trace_blocks);
         if (prof) prof->begin(K_TAIL);
         if (wide)
             hipLaunchKernelGGL(k_tail<true>, dim3(tail_grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg, counters,
-                               tail_claims, base, bounce, light_sampling);
+                               counters + tail_claim_index(max_bounces), base, bounce, light_sampling);
         else
             hipLaunchKernelGGL(k_tail<false>, dim3(tail_grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg, counters,
-                               tail_claims, base, bounce, light_sampling);
+                               counters + tail_claim_index(max_bounces), base, bounce, light_sampling);
         if (prof) prof->end(K_TAIL);
         return hipGetLastError();
     }
