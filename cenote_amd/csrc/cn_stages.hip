@@ -933,26 +933,36 @@ __global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu
     const uint32_t owner = __lane_id() & ~1u, mate = __lane_id() | 1u;
     // Items: the miss-queue entries [0, n_miss), then the hit-queue entries
     // [n_miss, n), one per lane pair. Pairs take items as they free up: a
-    // wave claims one item for each of its idle pairs with one atomic on one
+    // wave claims one item for each idle pair it has room for with one atomic on one
     // of QUEUE_SPLIT striped counters (stripe k deals items k, k + QUEUE_SPLIT,
     // ...), moving to a stripe with items left once its own runs out, so no
     // pair waits on the longest path of its wave while items remain. A pair
     // carries its path from bounce to bounce itself, in order.
     uint32_t stripe = (blockIdx.x * (TRAVERSAL_BLOCK / 64) + threadIdx.x / 64) % QUEUE_SPLIT;  // wave-uniform
     bool items_left = true;  // wave-uniform
+    // Few items go over many waves: a wave carries no more pairs at once than
+    // its share of all items. A launch's length is its longest path's, and a
+    // wave's bounce lasts as long as the longest walk of its pairs (the 2M-
+    // triangle scene's 28,000 paths 1.25 -> 0.92 ms from outside, 1.20 -> 1.00
+    // from inside; the veiled chart 0.56 -> 0.30; twice the share 1.10, 1.16
+    // and 0.29. The Cornell box, whose walks are short, 0.09 -> 0.11).
+    const uint32_t waves = gridDim.x * (TRAVERSAL_BLOCK / 64);
+    const uint32_t share = min(max(n / waves, 1u), 32u);
     bool live = false;  // the pair carries a path (the same in both lanes)
     uint32_t path = 0, b = 0;
     while (true) {
         const uint64_t idle = __ballot(!live && !helper);  // the idle pairs' owners
-        if (idle != 0 && items_left) {
-            const uint32_t want = __popcll(idle);
+        const uint32_t idle_pairs = __popcll(idle);
+        const uint32_t room = share - min(share, 32u - idle_pairs);
+        const uint32_t want = min(idle_pairs, room);
+        if (want != 0 && items_left) {
             const uint32_t leader = __ffsll((unsigned long long)idle) - 1;
             uint32_t c = 0;
             if (__lane_id() == leader) c = atomicAdd(&claims[stripe * COUNTER_STRIDE], want);
             c = __builtin_amdgcn_readlane(c, leader);
             if (!live) {
                 const uint32_t rank = __popcll(idle & ((1ull << owner) - 1));
-                const uint32_t i = stripe + QUEUE_SPLIT * (c + rank);
+                const uint32_t i = rank < want ? stripe + QUEUE_SPLIT * (c + rank) : n;
                 if (i < n_miss) {
                     const uint32_t entry = p.miss_queue[queue_slot(counters, bounce, Q_MISS, i, p.sub_capacity)];
                     if (!helper) miss_path(s, p, tg, entry, base, bounce, light_sampling);
