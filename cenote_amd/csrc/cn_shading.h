@@ -103,7 +103,7 @@ __device__ __forceinline__ float tab3(const float* t, uint32_t off, float x, flo
     return lerpf(tab2(t, off + 256u * i, 16, 16, x, y), tab2(t, off + 256u * j, 16, 16, x, y), fz - float(i));
 }
 
-__device__ __forceinline__ float ior_remap(float eta) { return sqrtf(fabsf(eta - 1.0f) / (eta + 1.0f)); }
+__device__ __forceinline__ float ior_remap(float eta) { return sqrt_n(div_n(fabsf(eta - 1.0f), eta + 1.0f)); }
 
 // --- EON diffuse (openpbr.slang:134-175) ----------------------------------------
 
@@ -113,21 +113,21 @@ __device__ __forceinline__ float fon_b() { return 2.0f / 3.0f - 28.0f / (15.0f *
 __device__ __forceinline__ float fon_albedo(float mu, float r) {
     const float g = 1.0f - mu;
     const float gOverPi = g * (0.0571085289f + g * (0.491881867f + g * (-0.332181442f + g * 0.0714429953f)));
-    return (1.0f + r * gOverPi) / (1.0f + fon_a() * r);
+    return div_n(1.0f + r * gOverPi, 1.0f + fon_a() * r);
 }
 
 __device__ __forceinline__ v3 eon_brdf(v3 rho, float r, v3 wi, v3 wo) {
     const float s = dot(wi, wo) - wi.z * wo.z;
-    const float sOverT = s > 0.0f ? s / fmaxf(wi.z, wo.z) : s;
-    const float A = 1.0f / (1.0f + fon_a() * r);
-    const v3 single = ((rho / PI_B) * A) * (1.0f + r * sOverT);
+    const float sOverT = s > 0.0f ? div_n(s, fmaxf(wi.z, wo.z)) : s;
+    const float A = rcp_n(1.0f + fon_a() * r);
+    const v3 single = (div_n(rho, PI_B) * A) * (1.0f + r * sOverT);
     const float albedoI = fon_albedo(wi.z, r);
     const float albedoO = fon_albedo(wo.z, r);
     const float albedoAvg = A * (1.0f + fon_b() * r);
-    const v3 rhoMulti = ((rho * rho) * albedoAvg) / (S3(1.0f) - rho * (1.0f - albedoAvg));
+    const v3 rhoMulti = div_n((rho * rho) * albedoAvg, S3(1.0f) - rho * (1.0f - albedoAvg));
     const float eps = 1e-7f;
-    const v3 multi = (((rhoMulti / PI_B) * fmaxf(eps, 1.0f - albedoO)) * fmaxf(eps, 1.0f - albedoI)) /
-                     fmaxf(eps, 1.0f - albedoAvg);
+    const v3 multi = div_n((div_n(rhoMulti, PI_B) * fmaxf(eps, 1.0f - albedoO)) * fmaxf(eps, 1.0f - albedoI),
+                           fmaxf(eps, 1.0f - albedoAvg));
     return single + multi;
 }
 
@@ -136,26 +136,25 @@ __device__ __forceinline__ v3 eon_brdf(v3 rho, float r, v3 wi, v3 wo) {
 __device__ __forceinline__ float ggx_d(float alpha, float hz) {
     const float a2 = alpha * alpha;
     const float denom = hz * hz * (a2 - 1.0f) + 1.0f;
-    return hz > 0.0f ? a2 / (PI_B * denom * denom) : 0.0f;
+    return hz > 0.0f ? div_n(a2, PI_B * denom * denom) : 0.0f;
 }
 
 __device__ __forceinline__ float smith_g1(float alpha, float vz) {
     const float a2 = alpha * alpha;
-    return 2.0f * fabsf(vz) / (fabsf(vz) + sqrtf(vz * vz * (1.0f - a2) + a2));
+    return div_n(2.0f * fabsf(vz), fabsf(vz) + sqrt_n(vz * vz * (1.0f - a2) + a2));
 }
 
 // Dupuy & Benyoub spherical-cap VNDF sampling (openpbr.slang:198-210).
 __device__ __forceinline__ v3 sample_vndf(v3 wo, float alpha, f2 u) {
-    const v3 woStd = normalize(V3(wo.x * alpha, wo.y * alpha, wo.z));
+    const v3 woStd = normalize_n(V3(wo.x * alpha, wo.y * alpha, wo.z));
     const float phi = 2.0f * PI_B * u.x;
     const float z = fmaf(1.0f - u.y, 1.0f + woStd.z, -woStd.z);
-    const float sinTheta = sqrtf(clampf(1.0f - z * z, 0.0f, 1.0f));
+    const float sinTheta = sqrt_n(clampf(1.0f - z * z, 0.0f, 1.0f));
     float sp, cp;
-    sp = sinf(phi);
-    cp = cosf(phi);
+    sincosf(phi, &sp, &cp);  // the bits of sinf and cosf, one argument reduction
     const v3 c = V3(sinTheta * cp, sinTheta * sp, z);
     const v3 hStd = c + woStd;
-    return normalize(V3(hStd.x * alpha, hStd.y * alpha, hStd.z));
+    return normalize_n(V3(hStd.x * alpha, hStd.y * alpha, hStd.z));
 }
 
 __device__ __forceinline__ float vndf_reflect_pdf(float alpha, v3 wo, v3 h) {
@@ -171,23 +170,23 @@ __device__ __forceinline__ v3 fresnel_schlick(v3 f0, float cosine) {
 __device__ __forceinline__ float fresnel_dielectric(float eta, float cosine) {
     const float mu = fabsf(cosine);
     const float sin2 = 1.0f - mu * mu;
-    const float cos2t = 1.0f - sin2 / (eta * eta);
+    const float cos2t = 1.0f - div_n(sin2, eta * eta);
     if (cos2t < 0.0f) return 1.0f;
-    const float t0 = sqrtf(cos2t);
+    const float t0 = sqrt_n(cos2t);
     const float t1 = eta * t0;
     const float t2 = eta * mu;
-    const float rs = (mu - t1) / (mu + t1);
-    const float rp = (t0 - t2) / (t0 + t2);
+    const float rs = div_n(mu - t1, mu + t1);
+    const float rp = div_n(t0 - t2, t0 + t2);
     return (rs * rs + rp * rp) / 2.0f;
 }
 
 __device__ __forceinline__ float fresnel_dielectric_avg(float eta) {
     if (eta < 1.0f) return 0.997118f + eta * (0.1014f - eta * (0.965241f + eta * 0.130607f));
-    return (eta - 1.0f) / (4.08567f + 1.00071f * eta);
+    return div_n(eta - 1.0f, 4.08567f + 1.00071f * eta);
 }
 
 __device__ __forceinline__ v3 fresnel_ms(v3 fss, float eAvg) {
-    return (fss * eAvg) / (S3(1.0f) - fss * (1.0f - eAvg));
+    return div_n(fss * eAvg, S3(1.0f) - fss * (1.0f - eAvg));
 }
 
 // --- the closure (openpbr.slang:295-587) -----------------------------------------
@@ -213,7 +212,7 @@ struct Closure {
 __device__ __forceinline__ v3 reflection_scale(const float* t, float rough, float mu, v3 fss) {
     const float e = fmaxf(1e-4f, tab2(t, T_GGX_E, 32, 32, rough, mu));
     const float eAvg = tab1(t, T_GGX_E_AVG, 32, rough);
-    return 1.0f + fresnel_ms(fss, eAvg) * ((1.0f - e) / e);
+    return 1.0f + fresnel_ms(fss, eAvg) * div_n(1.0f - e, e);
 }
 
 // openpbr.slang:357-363
@@ -225,13 +224,13 @@ __device__ __forceinline__ float dielectric_albedo(const float* t, float rough, 
 // openpbr.slang:371-384
 __device__ __forceinline__ v3 coat_darkening(const Mat& m, float rough, float mu, float baseFresnel) {
     const float fssCoat = fresnel_dielectric_avg(m.coatIor);
-    const float kRough = 1.0f - (1.0f - fssCoat) / (m.coatIor * m.coatIor);
+    const float kRough = 1.0f - div_n(1.0f - fssCoat, m.coatIor * m.coatIor);
     const float kSmooth = fresnel_dielectric(m.coatIor, mu);
     const float roughDiffuse = lerpf(1.0f, rough, saturate(m.specularWeight * baseFresnel));
     const float baseRough = lerpf(roughDiffuse, rough, m.metalness);
     const float k = lerpf(kSmooth, kRough, baseRough);
     const v3 baseAlbedo = vlerp(m.baseColor, S3(1.0f), (1.0f - m.metalness) * m.transmissionWeight);
-    const v3 darkened = (1.0f - k) / vmax(S3(1e-4f), 1.0f - baseAlbedo * k);
+    const v3 darkened = div_n(1.0f - k, vmax(S3(1e-4f), 1.0f - baseAlbedo * k));
     return vlerp(S3(1.0f), darkened, m.coatWeight * m.coatDarkening);
 }
 
@@ -249,22 +248,22 @@ __device__ inline Closure resolve_closure(const float* t, const Mat& m, v3 wo, b
     if (coated) {
         const float variance =
             fminf(1.0f, rough * rough * rough * rough + 2.0f * coatRough * coatRough * coatRough * coatRough);
-        rough = lerpf(rough, sqrtf(sqrtf(variance)), m.coatWeight);
+        rough = lerpf(rough, sqrt_n(sqrt_n(variance)), m.coatWeight);
     }
     c.alpha = rough * rough;
     c.coatAlpha = coatRough * coatRough;
 
     float etaS = fmaxf(m.specularIor, 1e-4f);
     if (coated) {
-        const float etaBc = m.coatIor > etaS ? m.coatIor / etaS : etaS / m.coatIor;
+        const float etaBc = m.coatIor > etaS ? div_n(m.coatIor, etaS) : div_n(etaS, m.coatIor);
         etaS = lerpf(etaS, etaBc, m.coatWeight);
     }
-    const float f0 = (etaS - 1.0f) * (etaS - 1.0f) / ((etaS + 1.0f) * (etaS + 1.0f));
-    const float weight = clampf(m.specularWeight, 0.0f, f0 > 1e-6f ? 1.0f / f0 : 0.0f);
+    const float f0 = div_n((etaS - 1.0f) * (etaS - 1.0f), (etaS + 1.0f) * (etaS + 1.0f));
+    const float weight = clampf(m.specularWeight, 0.0f, f0 > 1e-6f ? rcp_n(f0) : 0.0f);
     const float epsilon = signf(etaS - 1.0f) * sqrtf(weight * f0);
-    float eta = (1.0f + epsilon) / fmaxf(1e-3f, 1.0f - epsilon);
+    float eta = div_n(1.0f + epsilon, fmaxf(1e-3f, 1.0f - epsilon));
     if (fabsf(eta - 1.0f) < 1e-3f) eta = eta < 1.0f ? 1.0f - 1e-3f : 1.0f + 1e-3f;
-    c.eta = exiting ? 1.0f / eta : eta;
+    c.eta = exiting ? rcp_n(eta) : eta;
 
     c.fuzzA = 0.0f;
     c.fuzzB = 0.0f;
@@ -301,14 +300,14 @@ __device__ inline Closure resolve_closure(const float* t, const Mat& m, v3 wo, b
     float glassEta = c.eta;
     uint32_t glassOff = T_GLASS_E, glassAvgOff = T_GLASS_E_AVG;
     if (glassEta < 1.0f) {
-        glassEta = 1.0f / glassEta;
+        glassEta = rcp_n(glassEta);
         glassOff = T_GLASS_INV_E;
         glassAvgOff = T_GLASS_INV_E_AVG;
     }
     const float glassZ = ior_remap(glassEta);
     const float glassE = fmaxf(1e-4f, tab3(t, glassOff, rough, mu, glassZ));
     const float glassEAvg = tab2(t, glassAvgOff, 16, 16, rough, glassZ);
-    c.glassScale = 1.0f + fresnel_ms(c.glassTint, glassEAvg) * ((1.0f - glassE) / glassE);
+    c.glassScale = 1.0f + fresnel_ms(c.glassTint, glassEAvg) * div_n(1.0f - glassE, glassE);
 
     c.thinR = S3(0.0f);
     c.thinT = S3(0.0f);
@@ -318,40 +317,40 @@ __device__ inline Closure resolve_closure(const float* t, const Mat& m, v3 wo, b
     c.thinTShare = 0.0f;
     const bool thin = m.thinWalled != 0 && m.transmissionWeight > 0.0f;
     if (thin) {
-        const float thinEta = fmaxf(eta, 1.0f / eta);
+        const float thinEta = fmaxf(eta, rcp_n(eta));
         const float r1 = fresnel_dielectric(thinEta, mu);
         const float t1 = 1.0f - r1;
-        const float cos2t = fmaxf(0.0f, 1.0f - (1.0f - mu * mu) / (thinEta * thinEta));
+        const float cos2t = fmaxf(0.0f, 1.0f - div_n(1.0f - mu * mu, thinEta * thinEta));
         v3 absorb = S3(0.0f);
         if (cos2t > 0.0f) {
             const v3 tc = vclamp(m.transmissionColor, 1e-4f, 1.0f);
-            const float p = 1.0f / sqrtf(cos2t);
+            const float p = rcp_n(sqrt_n(cos2t));
             absorb = V3(powf(tc.x, p), powf(tc.y, p), powf(tc.z, p));
         }
         const v3 denom = vmax(S3(1e-4f), 1.0f - (absorb * absorb) * (r1 * r1));
-        c.thinT = (absorb * (t1 * t1)) / denom;
+        c.thinT = div_n(absorb * (t1 * t1), denom);
         c.thinR = r1 + c.thinT * (r1 * absorb);
         const float thinRough = clampf(
-            rough * sqrtf(3.4f * (thinEta - 1.0f) * (thinEta - 0.5f) * (thinEta - 0.5f) / (thinEta * thinEta * thinEta)),
+            rough * sqrt_n(div_n(3.4f * (thinEta - 1.0f) * (thinEta - 0.5f) * (thinEta - 0.5f), thinEta * thinEta * thinEta)),
             MIN_SPEC_ROUGH, 1.0f);
         c.thinAlpha = thinRough * thinRough;
         c.thinScaleR = reflection_scale(t, rough, mu, S3(1.0f)).x;
         c.thinScaleT = reflection_scale(t, thinRough, mu, S3(1.0f)).x;
-        const float total = mean3(c.thinR) + mean3(c.thinT);
-        c.thinTShare = total > 0.0f ? mean3(c.thinT) / total : 0.0f;
+        const float total = mean3_n(c.thinR) + mean3_n(c.thinT);
+        c.thinTShare = total > 0.0f ? div_n(mean3_n(c.thinT), total) : 0.0f;
     }
 
-    const float schlickS = saturate((c.specE - f0) / fmaxf(1e-4f, 1.0f - f0));
+    const float schlickS = saturate(div_n(c.specE - f0, fmaxf(1e-4f, 1.0f - f0)));
     const v3 metalE = vlerp(m.baseColor, S3(1.0f), schlickS);
-    const float glassTotal = thin ? mean3(c.thinR + c.thinT) : c.specE + (1.0f - c.specE) * mean3(c.glassTint);
+    const float glassTotal = thin ? mean3_n(c.thinR + c.thinT) : c.specE + (1.0f - c.specE) * mean3_n(c.glassTint);
     const float dielectricE = lerpf(c.specE, glassTotal, m.transmissionWeight);
-    const float baseAvg = mean3(c.baseWeight);
-    c.wFuzz = exiting ? 0.0f : m.fuzzWeight * c.fuzzR * mean3(m.fuzzColor);
+    const float baseAvg = mean3_n(c.baseWeight);
+    c.wFuzz = exiting ? 0.0f : m.fuzzWeight * c.fuzzR * mean3_n(m.fuzzColor);
     c.wCoat = exiting ? 0.0f : c.fuzzAtten * m.coatWeight * c.coatE;
-    c.wSpec = c.hasSpecular ? baseAvg * lerpf(dielectricE, mean3(metalE), m.metalness) : 0.0f;
+    c.wSpec = c.hasSpecular ? baseAvg * lerpf(dielectricE, mean3_n(metalE), m.metalness) : 0.0f;
     c.wDiffuse = exiting ? 0.0f
                          : baseAvg * (1.0f - m.metalness) * (1.0f - m.transmissionWeight) * (1.0f - c.specE) *
-                               mean3(m.baseColor);
+                               mean3_n(m.baseColor);
     if (exiting) c.wSpec = 1.0f;
     c.wTotal = c.wFuzz + c.wCoat + c.wSpec + c.wDiffuse;
 
@@ -381,7 +380,7 @@ __device__ __forceinline__ float aov_record_fraction(const Closure& c, uint32_t 
     else if (lobe == LOBE_SPECULAR) alpha = spec;
     else if (lobe == LOBE_TRANSMISSION) alpha = c.m.thinWalled != 0 ? thin : spec;
     else return 1.0f;
-    return saturate(sqrtf(alpha) / 0.15f);
+    return saturate(div_n(sqrt_n(alpha), 0.15f));
 }
 
 // openpbr.slang:614-622
@@ -395,15 +394,15 @@ __device__ __forceinline__ v3 aov_pass_tint(const Closure& c, uint32_t lobe) {
 __device__ __forceinline__ float sheen_density(const Closure& c, v3 w) {
     const float a = c.fuzzA, b = c.fuzzB;
     const float lenSqr = (a * w.x + b * w.z) * (a * w.x + b * w.z) + (a * w.y) * (a * w.y) + w.z * w.z;
-    const float ratio = a / lenSqr;
-    return fmaxf(w.z, 0.0f) * ratio * ratio / PI_B;
+    const float ratio = div_n(a, lenSqr);
+    return div_n(fmaxf(w.z, 0.0f) * ratio * ratio, PI_B);
 }
 
 __device__ __forceinline__ v3 align_to_view(v3 v, v3 wo, bool inverse) {
-    const float len = sqrtf(wo.x * wo.x + wo.y * wo.y);
+    const float len = sqrt_n(fmaxf(wo.x * wo.x + wo.y * wo.y, 1e-30f));  // (the floor lies below the cut)
     if (len < 1e-6f) return v;
-    const float cosPhi = wo.x / len;
-    const float sinPhi = (inverse ? -wo.y : wo.y) / len;
+    const float cosPhi = div_n(wo.x, len);
+    const float sinPhi = div_n(inverse ? -wo.y : wo.y, len);
     return V3(cosPhi * v.x + sinPhi * v.y, cosPhi * v.y - sinPhi * v.x, v.z);
 }
 
@@ -539,14 +538,14 @@ __device__ inline BsdfEval eval_with_pdf(const Closure& c, v3 wi, v3 wo) {
         if (!fOn && !pOn) return r;
         if (m.thinWalled != 0) {
             const v3 flipped = V3(wi.x, wi.y, -wi.z);
-            const v3 h = normalize(flipped + wo);
+            const v3 h = normalize_n(flipped + wo);
             const float D = ggx_d(c.thinAlpha, h.z), G1o = smith_g1(c.thinAlpha, wo.z);
             if (fOn) {
-                const float core = D * G1o * smith_g1(c.thinAlpha, flipped.z) / (4.0f * wo.z * flipped.z);
+                const float core = div_n(D * G1o * smith_g1(c.thinAlpha, flipped.z), 4.0f * wo.z * flipped.z);
                 r.f = ((c.baseWeight * glassShare) * c.thinT) * c.thinScaleT * core;
             }
             if (pOn) {
-                const float pdf = G1o * D / (4.0f * wo.z) * (1.0f - reflect_probability(c, 0.0f));
+                const float pdf = div_n(G1o * D, 4.0f * wo.z) * (1.0f - reflect_probability(c, 0.0f));
                 r.pdf = c.wSpec * pdf / c.wTotal;
             }
             return r;
@@ -554,7 +553,7 @@ __device__ inline BsdfEval eval_with_pdf(const Closure& c, v3 wi, v3 wo) {
         const v3 hU = wo + c.eta * wi;
         const float len2 = dot(hU, hU);
         if (len2 < 1e-9f) return r;
-        v3 h = hU / sqrtf(len2);
+        v3 h = div_n(hU, sqrt_n(len2));
         h = h.z >= 0.0f ? h : -h;
         const float cosVH = dot(h, wo);
         const float cosLH = dot(h, wi);
@@ -562,13 +561,13 @@ __device__ inline BsdfEval eval_with_pdf(const Closure& c, v3 wi, v3 wo) {
         const float f = fresnel_dielectric(c.eta, cosVH);
         const float D = ggx_d(c.alpha, h.z), G1o = smith_g1(c.alpha, wo.z);
         if (fOn) {
-            const float core = D * G1o * smith_g1(c.alpha, wi.z) * cosVH * (c.eta * c.eta) * fabsf(cosLH) /
-                               (wo.z * fabsf(wi.z) * len2);
+            const float core = div_n(D * G1o * smith_g1(c.alpha, wi.z) * cosVH * (c.eta * c.eta) * fabsf(cosLH),
+                                     wo.z * fabsf(wi.z) * len2);
             r.f = ((((c.baseWeight * glassShare) * (1.0f - f)) * c.glassTint) * c.glassScale) * core;
         }
         if (pOn) {
-            const float vndf = G1o * D * cosVH / wo.z;
-            const float jacobian = (c.eta * c.eta) * fabsf(cosLH) / len2;
+            const float vndf = div_n(G1o * D * cosVH, wo.z);
+            const float jacobian = div_n((c.eta * c.eta) * fabsf(cosLH), len2);
             const float pdf = vndf * jacobian * (1.0f - reflect_probability(c, f));
             r.pdf = c.wSpec * pdf / c.wTotal;
         }
@@ -578,7 +577,7 @@ __device__ inline BsdfEval eval_with_pdf(const Closure& c, v3 wi, v3 wo) {
     const bool coatF = m.coatWeight > 0.0f && !c.exiting, coatP = pdfOn && c.wCoat > 0.0f;
     const bool specF = c.hasSpecular, specP = pdfOn && c.wSpec > 0.0f;
     const float density = (fuzzF || fuzzP) ? sheen_density(c, align_to_view(wi, wo, false)) : 0.0f;
-    const v3 h = normalize(wi + wo);
+    const v3 h = normalize_n(wi + wo);
     const float cosVH = dot(h, wo);
     float coatD = 0.0f, coatG1o = 0.0f, specD = 0.0f, specG1o = 0.0f, fd = 0.0f;
     if (coatF || coatP) {
@@ -593,15 +592,15 @@ __device__ inline BsdfEval eval_with_pdf(const Closure& c, v3 wi, v3 wo) {
 
     // eval_bsdf's reflection branch
     v3 result = S3(0.0f);
-    if (fuzzF) result = result + ((m.fuzzWeight * m.fuzzColor) * c.fuzzR) * density / wi.z;
+    if (fuzzF) result = result + div_n(((m.fuzzWeight * m.fuzzColor) * c.fuzzR) * density, wi.z);
     if (coatF) {
         const float coatFresnel = fresnel_dielectric(m.coatIor, cosVH);
-        const float core = coatD * coatG1o * smith_g1(c.coatAlpha, wi.z) / (4.0f * wo.z * wi.z);
+        const float core = div_n(coatD * coatG1o * smith_g1(c.coatAlpha, wi.z), 4.0f * wo.z * wi.z);
         result = result + S3(c.fuzzAtten * m.coatWeight * coatFresnel * c.coatScale * core);
     }
     v3 base = S3(0.0f);
     if (specF) {  // base_reflection
-        const float core = specD * specG1o * smith_g1(c.alpha, wi.z) / (4.0f * wo.z * wi.z);
+        const float core = div_n(specD * specG1o * smith_g1(c.alpha, wi.z), 4.0f * wo.z * wi.z);
         if (c.exiting) {
             base = S3(core * fd) * c.glassScale;
         } else {
@@ -622,9 +621,9 @@ __device__ inline BsdfEval eval_with_pdf(const Closure& c, v3 wi, v3 wo) {
     if (pdfOn) {
         float pdf = 0.0f;
         if (c.wFuzz > 0.0f) pdf += c.wFuzz * density;
-        if (c.wCoat > 0.0f) pdf += c.wCoat * (coatG1o * coatD / (4.0f * wo.z));
-        if (c.wSpec > 0.0f) pdf += c.wSpec * (specG1o * specD / (4.0f * wo.z)) * reflect_probability(c, fd);
-        if (c.wDiffuse > 0.0f) pdf += c.wDiffuse * wi.z / PI_B;
+        if (c.wCoat > 0.0f) pdf += c.wCoat * div_n(coatG1o * coatD, 4.0f * wo.z);
+        if (c.wSpec > 0.0f) pdf += c.wSpec * div_n(specG1o * specD, 4.0f * wo.z) * reflect_probability(c, fd);
+        if (c.wDiffuse > 0.0f) pdf += div_n(c.wDiffuse * wi.z, PI_B);
         r.pdf = pdf / c.wTotal;
     }
     return r;
@@ -639,59 +638,55 @@ struct BsdfSample {
 // openpbr.slang:821-884, up to the pdf: draws the scattered direction and
 // lobe into `r` (pdf left 0) and returns whether one was drawn; the pdf of a
 // drawn direction is bsdf_pdf(c, r.wi, wo), which eval_with_pdf also gives.
+//
+// The lobe is settled first, with the roughness its half vector is drawn
+// with, so that a wave draws every microfacet lobe's half vector in one piece
+// of code, and both cosine-weighted lobes' disk in another.
 __device__ inline bool sample_bsdf_direction(const Closure& c, v3 wo, float uLobe, f2 u, BsdfSample& r) {
     r = BsdfSample{V3(0.0f, 0.0f, 1.0f), 0.0f, LOBE_DIFFUSE};
     if (c.wTotal <= 0.0f) return false;
     const float pick = uLobe * c.wTotal;
-    v3 wi;
-    if (pick < c.wFuzz) {
-        r.lobe = LOBE_FUZZ;
-        const float rr = sqrtf(u.x);
-        const float phi = 2.0f * PI_B * u.y;
-        const float dx = rr * cosf(phi), dy = rr * sinf(phi);
-        const float diskZ = sqrtf(fmaxf(0.0f, 1.0f - (dx * dx + dy * dy)));
-        const v3 wiStd = normalize(V3(dx - diskZ * c.fuzzB, dy, diskZ * c.fuzzA));
-        wi = align_to_view(wiStd, wo, true);
-    } else if (pick < c.wFuzz + c.wCoat) {
-        r.lobe = LOBE_COAT;
-        const v3 h = sample_vndf(wo, c.coatAlpha, u);
-        wi = (2.0f * dot(wo, h)) * h - wo;
-    } else if (pick < c.wFuzz + c.wCoat + c.wSpec) {
-        const float uBranch = (pick - c.wFuzz - c.wCoat) / fmaxf(1e-6f, c.wSpec);
-        if (c.m.thinWalled != 0) {
-            if (uBranch < reflect_probability(c, 0.0f)) {
-                r.lobe = LOBE_SPECULAR;
-                const v3 h = sample_vndf(wo, c.alpha, u);
-                wi = (2.0f * dot(wo, h)) * h - wo;
-            } else {
-                r.lobe = LOBE_TRANSMISSION;
-                const v3 h = sample_vndf(wo, c.thinAlpha, u);
-                const v3 refl = (2.0f * dot(wo, h)) * h - wo;
-                wi = V3(refl.x, refl.y, -refl.z);
-            }
+    const bool fuzz = pick < c.wFuzz;
+    const bool coat = !fuzz && pick < c.wFuzz + c.wCoat;
+    const bool spec = !fuzz && !coat && pick < c.wFuzz + c.wCoat + c.wSpec;
+    if (coat || spec) {
+        const bool thin = spec && c.m.thinWalled != 0;
+        const float uBranch = div_n(pick - c.wFuzz - c.wCoat, fmaxf(1e-6f, c.wSpec));
+        bool through = thin && !(uBranch < reflect_probability(c, 0.0f));
+        // (read unconditionally and pinned, as in aov_record_fraction)
+        float coatAlpha = c.coatAlpha, specAlpha = c.alpha, thinAlpha = c.thinAlpha;
+        asm("" : "+v"(coatAlpha), "+v"(specAlpha), "+v"(thinAlpha));
+        const v3 h = sample_vndf(wo, coat ? coatAlpha : through ? thinAlpha : specAlpha, u);
+        if (spec && !thin) through = !(uBranch < reflect_probability(c, fresnel_dielectric(c.eta, dot(h, wo))));
+        r.lobe = coat ? LOBE_COAT : through ? LOBE_TRANSMISSION : LOBE_SPECULAR;
+        const v3 refl = (2.0f * dot(wo, h)) * h - wo;
+        if (!through) {
+            r.wi = refl;
+        } else if (thin) {
+            r.wi = V3(refl.x, refl.y, -refl.z);
         } else {
-            const v3 h = sample_vndf(wo, c.alpha, u);
-            const float f = fresnel_dielectric(c.eta, dot(h, wo));
-            if (uBranch < reflect_probability(c, f)) {
-                r.lobe = LOBE_SPECULAR;
-                wi = (2.0f * dot(wo, h)) * h - wo;
-            } else {
-                r.lobe = LOBE_TRANSMISSION;
-                // refractDirection, openpbr.slang:270-277
-                const float cc = dot(wo, h);
-                const float cos2t = 1.0f - (1.0f - cc * cc) / (c.eta * c.eta);
-                if (cos2t <= 0.0f) return false;
-                wi = h * (cc / c.eta - sqrtf(cos2t)) - wo / c.eta;
-            }
+            // refractDirection, openpbr.slang:270-277
+            const float cc = dot(wo, h);
+            const float cos2t = 1.0f - div_n(1.0f - cc * cc, c.eta * c.eta);
+            if (cos2t <= 0.0f) return false;
+            r.wi = h * (div_n(cc, c.eta) - sqrt_n(cos2t)) - div_n(wo, c.eta);
         }
-    } else {
-        r.lobe = LOBE_DIFFUSE;
-        // sampleCosineHemisphere, openpbr.slang:170-175
-        const float rr = sqrtf(u.x);
-        const float phi = 2.0f * PI_B * u.y;
-        wi = V3(rr * cosf(phi), rr * sinf(phi), sqrtf(1.0f - u.x));
+        return true;
     }
-    r.wi = wi;
+    const float rr = sqrt_n(u.x);
+    const float phi = 2.0f * PI_B * u.y;
+    float sp, cp;
+    sincosf(phi, &sp, &cp);
+    const float dx = rr * cp, dy = rr * sp;
+    if (fuzz) {
+        r.lobe = LOBE_FUZZ;
+        const float diskZ = sqrt_n(fmaxf(0.0f, 1.0f - (dx * dx + dy * dy)));
+        const v3 wiStd = normalize_n(V3(dx - diskZ * c.fuzzB, dy, diskZ * c.fuzzA));
+        r.wi = align_to_view(wiStd, wo, true);
+    } else {
+        // sampleCosineHemisphere, openpbr.slang:170-175
+        r.wi = V3(dx, dy, sqrt_n(1.0f - u.x));
+    }
     return true;
 }
 
@@ -701,7 +696,7 @@ struct Frame {
 };
 __device__ __forceinline__ Frame make_frame(v3 n) {
     const float s = n.z >= 0.0f ? 1.0f : -1.0f;
-    const float a = -1.0f / (s + n.z);
+    const float a = -rcp_n(s + n.z);
     const float m = n.x * n.y * a;
     return {V3(1.0f + s * n.x * n.x * a, s * m, -s * n.x), V3(m, s + n.y * n.y * a, -n.y), n};
 }
@@ -745,7 +740,7 @@ __device__ __forceinline__ v3 env_bilinear(const SceneView& s, float u, float v)
 
 // environment.slang:74-78
 __device__ __forceinline__ f2 uv_from_direction(v3 d) {
-    return {0.5f + atan2f(d.x, -d.z) / (2.0f * PI_K), acosf(clampf(d.y, -1.0f, 1.0f)) / PI_K};
+    return {0.5f + div_n(atan2f(d.x, -d.z), 2.0f * PI_K), div_n(acosf(clampf(d.y, -1.0f, 1.0f)), PI_K)};
 }
 
 __device__ __forceinline__ v3 env_radiance(const SceneView& s, v3 d) {
@@ -772,7 +767,7 @@ __device__ __forceinline__ void sample_cdf(const float* __restrict__ cdf, const 
     const float width = cdf[lo + 1] - cdf[lo];
     const float frac = width > 0.0f ? (u - cdf[lo]) / width : 0.0f;
     *index = lo;
-    *position = (float(lo) + frac) / float(count);
+    *position = div_n(float(lo) + frac, float(count));
 }
 
 struct EnvSample {
@@ -788,12 +783,13 @@ __device__ inline EnvSample env_sample(const SceneView& s, f2 u) {
     sample_cdf(s.env_conditional + row * (s.env_width + 1),
                s.env_conditional_guide + row * (s.env_conditional_buckets + 1), s.env_conditional_buckets,
                s.env_width, u.y, &col, &uu);
-    const float sinTheta = sinf(PI_K * v);
     const float phi = 2.0f * PI_K * (uu - 0.5f);
     const float theta = PI_K * v;
-    const float st = sinf(theta);
+    float sinTheta, cosTheta, sinPhi, cosPhi;
+    sincosf(theta, &sinTheta, &cosTheta);
+    sincosf(phi, &sinPhi, &cosPhi);
     EnvSample e;
-    e.direction = V3(st * sinf(phi), cosf(theta), -st * cosf(phi));
+    e.direction = V3(sinTheta * sinPhi, cosTheta, -sinTheta * cosPhi);
     e.radiance = env_bilinear(s, uu, v);
     e.pdf = sinTheta > 0.0f ? s.env_pdfs[row * s.env_width + col] / (2.0f * PI_K * PI_K * sinTheta) : 0.0f;
     return e;
@@ -801,12 +797,12 @@ __device__ inline EnvSample env_sample(const SceneView& s, f2 u) {
 
 // environment.slang:110-119
 __device__ __forceinline__ float env_pdf(const SceneView& s, v3 d) {
-    const float sinTheta = sqrtf(fmaxf(0.0f, 1.0f - d.y * d.y));
+    const float sinTheta = sqrt_n(fmaxf(0.0f, 1.0f - d.y * d.y));
     if (sinTheta <= 0.0f) return 0.0f;
     const f2 uv = uv_from_direction(d);
     const uint32_t col = min(uint32_t(uv.x * float(s.env_width)), s.env_width - 1);
     const uint32_t row = min(uint32_t(uv.y * float(s.env_height)), s.env_height - 1);
-    return s.env_pdfs[row * s.env_width + col] / (2.0f * PI_K * PI_K * sinTheta);
+    return div_n(s.env_pdfs[row * s.env_width + col], 2.0f * PI_K * PI_K * sinTheta);
 }
 
 // lights.slang:42-44
@@ -851,7 +847,7 @@ __device__ inline LightConnection sample_lights(const SceneView& s, float u, f2 
     c.instance = __float_as_uint(r4.w);
     c.primitive = r5.y;
     if (kind == LIGHT_KIND_TRIANGLE) {
-        const float su = sqrtf(uPoint.x);
+        const float su = sqrt_n(uPoint.x);
         const float b1 = 1.0f - su, b2 = uPoint.y * su;
         const v3 position = (anchor + b1 * edge1) + b2 * edge2;
         const v3 delta = position - from;

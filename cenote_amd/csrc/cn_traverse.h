@@ -110,7 +110,7 @@ __device__ __forceinline__ Stack make_stack(uint32_t* lds_stack, uint32_t* spill
 }
 
 __device__ __forceinline__ float safe_rcp(float x) {
-    return 1.0f / (fabsf(x) < 1e-20f ? copysignf(1e-20f, x) : x);
+    return rcp_n(fabsf(x) < 1e-20f ? copysignf(1e-20f, x) : x);
 }
 
 // Watertight ray/triangle test (Woop, Benthin & Wald, JCGT 2(1), 2013),
@@ -144,10 +144,13 @@ __device__ __forceinline__ Ray make_ray(v3 o, v3 d) {
         m = ay;
     }
     if (az > m) kz = 2;
+    // d.kz is at least half of a unit direction, so its reciprocal above is
+    // the one the quotients need.
     const float dz = kz == 0 ? d.x : kz == 1 ? d.y : d.z;
+    const float y = kz == 0 ? w.ix : kz == 1 ? w.iy : w.iz;
     w.kz = kz;
-    w.Sx = (kz == 0 ? d.y : kz == 1 ? d.z : d.x) / dz;
-    w.Sy = (kz == 0 ? d.z : kz == 1 ? d.x : d.y) / dz;
+    w.Sx = div_by(kz == 0 ? d.y : kz == 1 ? d.z : d.x, dz, y);
+    w.Sy = div_by(kz == 0 ? d.z : kz == 1 ? d.x : d.y, dz, y);
     return w;
 }
 
@@ -179,7 +182,9 @@ __device__ __forceinline__ bool hit_triangle(const Ray& w, v3 v0, v3 v1, v3 v2, 
     Bz = Sz * Bz;
     Cz = Sz * Cz;
     const float T = U * Az + Vv * Bz + W * Cz;
-    const float rcp = 1.0f / det;
+    // (a determinant beyond rcp_n's range takes the operator)
+    float rcp = rcp_step(det);
+    if (!(fabsf(det) >= 0x1p-125f && fabsf(det) <= 0x1p125f)) rcp = 1.0f / det;
     const float t = T * rcp;
     if (!(t >= 0.0f) || !(t <= tmax)) return false;
     *t_out = t;
