@@ -1355,7 +1355,43 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_packet_nodes(const BvhNode4Q* _
     out[i] = p;
 }
 
+// One triangle per thread, its corners gathered from the pooled vertices.
+__global__ __launch_bounds__(BUILD_BLOCK) void k_mesh_triangles(const float* __restrict__ positions,
+                                                                const float* __restrict__ normals,
+                                                                const uint32_t* __restrict__ indices, uint32_t count,
+                                                                MeshTriangle* __restrict__ out) {
+    for (uint32_t i = blockIdx.x * BUILD_BLOCK + threadIdx.x; i < count; i += gridDim.x * BUILD_BLOCK) {
+        const size_t i0 = 3 * size_t(indices[3 * size_t(i)]), i1 = 3 * size_t(indices[3 * size_t(i) + 1]),
+                     i2 = 3 * size_t(indices[3 * size_t(i) + 2]);
+        MeshTriangle t;
+        t.a = make_float4(positions[i0], positions[i0 + 1], positions[i0 + 2], normals[i0]);
+        t.b = make_float4(positions[i1], positions[i1 + 1], positions[i1 + 2], normals[i0 + 1]);
+        t.c = make_float4(positions[i2], positions[i2 + 1], positions[i2 + 2], normals[i0 + 2]);
+        t.d = make_float4(normals[i1], normals[i1 + 1], normals[i1 + 2], normals[i2]);
+        t.e = make_float4(normals[i2 + 1], normals[i2 + 2], 0.0f, 0.0f);
+        out[i] = t;
+    }
+}
+
 }  // namespace
+
+hipError_t build_mesh_triangles(const float* positions, const float* normals, size_t vertices,
+                                const uint32_t* indices, size_t triangles, MeshTriangle* out) {
+    if (triangles == 0) return hipSuccess;
+    Scratch s;
+    float* d_positions = s.get<float>(3 * vertices);
+    float* d_normals = s.get<float>(3 * vertices);
+    uint32_t* d_indices = s.get<uint32_t>(3 * triangles);
+    if (!d_positions || !d_normals || !d_indices) return hipErrorOutOfMemory;
+    hipError_t e = hipMemcpy(d_positions, positions, 12 * vertices, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(d_normals, normals, 12 * vertices, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(d_indices, indices, 12 * triangles, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_mesh_triangles, dim3(blocks_for(triangles)), dim3(BUILD_BLOCK), 0, nullptr, d_positions,
+                       d_normals, d_indices, uint32_t(triangles), out);
+    e = hipGetLastError();
+    return e == hipSuccess ? hipDeviceSynchronize() : e;
+}
 
 bool decode_packet_nodes(const BvhNode4Q* nodes, uint32_t count, BvhNode4P* out, std::string* error) {
     if (count == 0) return true;

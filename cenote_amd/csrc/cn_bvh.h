@@ -79,6 +79,12 @@ bool build_bvh_device(const std::vector<WorldTriangle>& input, uint32_t max_stac
 bool patch_triangle_flags(BvhTriangle* tris, uint32_t count, const uint32_t* instance_flags, uint32_t instances,
                           std::string* error);
 
+// Gathers the pooled mesh triangles hit reconstruction reads, on the device,
+// from pooled vertices (host memory, packed xyz positions and normals) and
+// pool-wide vertex indices into `triangles` device records.
+hipError_t build_mesh_triangles(const float* positions, const float* normals, size_t vertices,
+                                const uint32_t* indices, size_t triangles, MeshTriangle* out);
+
 // The packet walk's 128-byte nodes (BvhNode4P) from the device's quantized
 // ones, node for node, on the device (the same boxes, planes decoded).
 bool decode_packet_nodes(const BvhNode4Q* nodes, uint32_t count, BvhNode4P* out, std::string* error);

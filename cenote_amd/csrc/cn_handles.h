@@ -116,8 +116,7 @@ struct cn_scene {
     cn::DevBuf<cn::InstanceRecord> instances;
     cn::DevBuf<cn_material> materials;
     cn::DevBuf<cn_light_record> lights;
-    cn::DevBuf<float> positions, normals;
-    cn::DevBuf<uint32_t> indices;
+    cn::DevBuf<cn::MeshTriangle> mesh_tris;
     cn::DevBuf<float4> env_texels;
     cn::DevBuf<float> env_marginal, env_conditional, env_pdfs;
     cn::DevBuf<uint32_t> env_marginal_guide, env_conditional_guide;

@@ -161,6 +161,15 @@ struct alignas(16) BvhTriangle {
 };
 static_assert(sizeof(BvhTriangle) == 48, "three dwordx4 fetches per triangle");
 
+// One triangle of a mesh in object space as hit reconstruction reads it:
+// corner positions and corner normals, gathered from the mesh's vertices once
+// at scene creation. A hit fetches 80 consecutive bytes (five dwordx4, one or
+// two lines) instead of its three indices and then six scattered vertices.
+struct alignas(16) MeshTriangle {
+    float4 a, b, c, d, e;  // v0, n0.x | v1, n0.y | v2, n0.z | n1, n2.x | n2.y, n2.z, -, -
+};
+static_assert(sizeof(MeshTriangle) == 80, "five dwordx4 fetches per hit");
+
 constexpr uint32_t TRI_NON_OPAQUE = 1u;
 constexpr uint32_t TRI_CLASS_SHIFT = 16;  // bits 16..20: the instance material's class
 
@@ -174,18 +183,16 @@ static_assert(CN_POOL_CAPACITY_MAX <= (1u << HIT_PATH_BITS), "path indices fit a
 // --- Scene records -----------------------------------------------------------
 
 // Per instance, 128 bytes: the GeometryRecord of scene/mod.rs:104-123 with
-// the mesh pointers replaced by offsets into the scene's pooled vertex and
-// index arrays.
+// the mesh pointers replaced by an offset into the scene's pooled triangles.
 struct alignas(16) InstanceRecord {
     float4 o2w[3];   // rows of the object-to-world transform
     float4 w2o[3];   // rows of its inverse
     uint32_t light;  // first light record, or LIGHT_NONE
-    uint32_t vertex_base;
-    uint32_t index_base;  // in triangles
+    uint32_t triangle_base;  // the mesh's first triangle in the pooled array
     uint32_t flags;       // bits 0..7 = visibility mask, bit 8 = opaque
     uint32_t material_class;     // which lobes the closure has (material-sorted shading)
     int32_t log2_transmittance;  // log2(1 - opacity) in 2^-24 units (log2_transmittance_fixed)
-    uint32_t pad[2];
+    uint32_t pad[3];
 };
 static_assert(sizeof(InstanceRecord) == 128, "two dwordx4 lines per instance");
 
@@ -201,9 +208,7 @@ struct SceneView {
     const InstanceRecord* instances;
     const cn_material* materials;
     const cn_light_record* lights;
-    const float* positions;  // pooled object-space xyz
-    const float* normals;    // pooled object-space xyz
-    const uint32_t* indices; // pooled, mesh-local vertex indices
+    const MeshTriangle* mesh_tris;  // pooled object-space triangles
     const float* tables;     // BSDF tables (16,928 floats)
     const float4* env_texels;
     const float* env_marginal;

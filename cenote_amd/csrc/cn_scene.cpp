@@ -137,8 +137,7 @@ int prep_instances(const cn_scene_desc* desc, const MeshPool& pool, std::vector<
         const cn_mesh& mesh = desc->meshes[inst.mesh];
         const uint32_t mask = inst.camera_visible ? MASK_ALL : (MASK_ALL & ~MASK_CAMERA);
         const bool opaque = inst.material.opacity >= 1.0f;
-        r.vertex_base = pool.vbase[inst.mesh];
-        r.index_base = pool.ibase[inst.mesh];
+        r.triangle_base = pool.ibase[inst.mesh];
         r.flags = mask | (opaque ? 0x100u : 0u);
         r.material_class = material_class(inst.material);
         r.log2_transmittance = opaque ? 0 : log2_transmittance_fixed(inst.material.opacity);
@@ -224,9 +223,7 @@ void refresh_view(cn_scene* scene) {
     v.instances = scene->instances.ptr;
     v.materials = scene->materials.ptr;
     v.lights = scene->lights.ptr;
-    v.positions = scene->positions.ptr;
-    v.normals = scene->normals.ptr;
-    v.indices = scene->indices.ptr;
+    v.mesh_tris = scene->mesh_tris.ptr;
     v.tables = scene->ctx->tables.ptr;
     v.env_texels = scene->env_texels.ptr;
     v.env_marginal = scene->env_marginal.ptr;
@@ -278,7 +275,9 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
         const cn_mesh& mesh = desc->meshes[m];
         std::memcpy(&positions[3 * size_t(pool.vbase[m])], mesh.positions, 12 * size_t(mesh.vertex_count));
         std::memcpy(&normals[3 * size_t(pool.vbase[m])], mesh.normals, 12 * size_t(mesh.vertex_count));
-        std::memcpy(&indices[3 * size_t(pool.ibase[m])], mesh.indices, 12 * size_t(mesh.triangle_count));
+        uint32_t* const out = indices.data() + 3 * size_t(pool.ibase[m]);
+        const uint32_t base = pool.vbase[m];
+        for (size_t k = 0; k < 3 * size_t(mesh.triangle_count); ++k) out[k] = base + mesh.indices[k];
     }
 
     Bvh4 bvh;
@@ -304,9 +303,9 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
         return fail(CN_E_SCENE, "%s", error.c_str());
     CN_HIP(scene->instances.upload(records.data(), records.size()));
     CN_HIP(scene->materials.upload(materials.data(), materials.size()));
-    CN_HIP(scene->positions.upload(positions.data(), positions.size()));
-    CN_HIP(scene->normals.upload(normals.data(), normals.size()));
-    CN_HIP(scene->indices.upload(indices.data(), indices.size()));
+    CN_HIP(scene->mesh_tris.alloc(pool.triangles));
+    CN_HIP(build_mesh_triangles(positions.data(), normals.data(), pool.vertices, indices.data(), pool.triangles,
+                                scene->mesh_tris.ptr));
     if (int e = install_lights(scene, std::move(emitters), desc->delta_lights, desc->delta_light_count)) return e;
     if (int e = install_environment(scene, desc->environment)) return e;
     scene->host_records = std::move(records);

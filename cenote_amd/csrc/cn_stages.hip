@@ -507,16 +507,13 @@ struct Spawn {
     bool frontFace;
 };
 
-__device__ __forceinline__ v3 load3(const float* a, uint32_t v) { return V3(a[3 * v], a[3 * v + 1], a[3 * v + 2]); }
-
 // shade_surface.slang:96-181: the hit rebuilt from the object-space mesh,
 // offset along the geometric normal by a rigorous bound on its own
 // reconstruction error (van Antwerpen 2023).
 __device__ inline Spawn spawn_point(const SceneView& s, const InstanceRecord& inst, uint32_t prim, float bx, float by,
                                     v3 rayDirection) {
-    const uint32_t* idx = s.indices + 3u * (inst.index_base + prim);
-    const uint32_t i0 = inst.vertex_base + idx[0], i1 = inst.vertex_base + idx[1], i2 = inst.vertex_base + idx[2];
-    const v3 v0 = load3(s.positions, i0), v1 = load3(s.positions, i1), v2 = load3(s.positions, i2);
+    const MeshTriangle tri = s.mesh_tris[inst.triangle_base + prim];
+    const v3 v0 = xyz(tri.a), v1 = xyz(tri.b), v2 = xyz(tri.c);
     const float4 a0 = inst.o2w[0], a1 = inst.o2w[1], a2 = inst.o2w[2];
     const float4 w0 = inst.w2o[0], w1 = inst.w2o[1], w2 = inst.w2o[2];
 
@@ -552,7 +549,7 @@ __device__ inline Spawn spawn_point(const SceneView& s, const InstanceRecord& in
     Spawn sp;
     sp.frontFace = dot(wldNormal, rayDirection) < 0.0f;
     if (dot(wldNormal, rayDirection) > 0.0f) wldNormal = -wldNormal;
-    const v3 n0 = load3(s.normals, i0), n1 = load3(s.normals, i1), n2 = load3(s.normals, i2);
+    const v3 n0 = V3(tri.a.w, tri.b.w, tri.c.w), n1 = xyz(tri.d), n2 = V3(tri.d.w, tri.e.x, tri.e.y);
     const v3 objShading = (n0 + bx * (n1 - n0)) + by * (n2 - n0);
     v3 shading = normalize((r0 * objShading.x + r1 * objShading.y) + r2 * objShading.z);
     if (dot(shading, wldNormal) < 0.0f) shading = -shading;
