@@ -12,8 +12,9 @@
 //     32-bin histograms on three axes), each range's split decided by one
 //     workgroup from those device-resident bins, then a stable scatter
 //     (per-chunk counts, per-range running sums, in-chunk scans);
-//   * every remaining range: one 256-lane workgroup builds its whole subtree
-//     in LDS, depth first, smaller child first;
+//   * every remaining range: one 256-lane workgroup splits it in LDS, depth
+//     first, smaller child first, down to ranges of at most WAVE_TASK;
+//   * those, each by one wave that holds its triangles in its lanes;
 //   * the collapse to 4-wide and 8-wide nodes, in the host collapse's
 //     preorder numbering, and their quantization.
 //
@@ -37,6 +38,8 @@ constexpr uint32_t BUILD_BLOCK = 256;
 constexpr uint32_t CHUNK = 8192;       // triangles per workgroup in the device-wide passes
 constexpr uint32_t SMALL_TASK = 2048;  // ranges at most this large are built by one workgroup
 constexpr uint32_t SMALL_STACK = 32;   // ample: smaller-first keeps it under log2(SMALL_TASK) + 1
+constexpr uint32_t WAVE_TASK = 64;     // ranges at most this large are built by one wave, a triangle a lane
+static_assert(WAVE_TASK >= BVH_LEAF_SIZE && WAVE_TASK < SMALL_TASK, "only a wave makes leaves");
 
 // Floats as order-preserving unsigned integers, so integer atomic min/max
 // fold float bounds exactly.
@@ -327,7 +330,8 @@ enum : uint32_t {
     S_CHUNKS = 7,    // chunks of the current level
     S_WIDE = 8,      // wide nodes allocated (collapse)
     S_LIST = 9,      // collapse list entries appended
-    S_WORDS = 10
+    S_WAVE = 10,     // wave tasks appended
+    S_WORDS = 11
 };
 
 // One level's chunk list (per big task, CHUNK-triangle chunks in range
@@ -563,11 +567,16 @@ __global__ void k_level_advance(uint32_t* state) {
 
 // --- subtrees: ranges of at most SMALL_TASK triangles --------------------------
 
-// One workgroup builds the whole subtree of one small range, depth first,
-// smaller child first, with the range's order held in LDS; bounds fold by
-// wave shuffles and every split is decided by the whole workgroup.
+// One workgroup splits one small range, depth first, smaller child first,
+// with the range's order held in LDS, down to ranges of at most WAVE_TASK
+// triangles, whose nodes it lists for k_wave_build (their range left in
+// first and count); bounds fold by wave shuffles and every split is decided
+// by the whole workgroup. A split costs some 17 us of barriers and dependent
+// gathers whatever the range's size, which is why it stops early: down to
+// the leaves this took 25.6 ms for a million triangles.
 __global__ __launch_bounds__(BUILD_BLOCK) void k_small_build(const Task* __restrict__ tasks, const uint32_t* counts,
                                                              PrimArrays p, uint32_t* order, BinaryNode* nodes,
+                                                             uint32_t* wave_list, uint32_t wave_capacity,
                                                              uint32_t* state) {
     __shared__ uint32_t ord[SMALL_TASK];
     __shared__ uint32_t tmp[SMALL_TASK];
@@ -581,8 +590,7 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_small_build(const Task* __restr
     __shared__ Decision dec;
     __shared__ uint32_t stack_b[SMALL_STACK], stack_e[SMALL_STACK], stack_n[SMALL_STACK];
     __shared__ uint32_t sp, cur_b, cur_e, cur_node, left;
-    __shared__ int live_leaf;  // 1: make a leaf
-    __shared__ int by_bin;     // 1: partition by bin, 0: by index
+    __shared__ int by_bin;  // 1: partition by bin, 0: by index
     __shared__ int axis, split;
     __shared__ float cb_lo[3], cb_scale[3];
     __shared__ int cb_live[3];
@@ -592,11 +600,26 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_small_build(const Task* __restr
     const Task t = tasks[blockIdx.x];
     const uint32_t n = t.end - t.begin;
     for (uint32_t i = threadIdx.x; i < n; i += BUILD_BLOCK) ord[i] = order[t.begin + i];
+    // Thread 0's: a range goes to the stack, or, once small, to the wave list.
+    const auto place = [&](uint32_t b, uint32_t e, uint32_t node) {
+        if (e - b <= WAVE_TASK) {
+            nodes[node].first = t.begin + b;
+            nodes[node].count = e - b;
+            const uint32_t at = atomicAdd(&state[S_WAVE], 1u);
+            if (at < wave_capacity) wave_list[at] = node;
+            else atomicOr(&state[S_OVERFLOW], 16u);
+        } else if (sp < SMALL_STACK) {
+            stack_b[sp] = b;
+            stack_e[sp] = e;
+            stack_n[sp] = node;
+            ++sp;
+        } else {
+            atomicOr(&state[S_OVERFLOW], 16u);
+        }
+    };
     if (threadIdx.x == 0) {
-        sp = 1;
-        stack_b[0] = 0;
-        stack_e[0] = n;
-        stack_n[0] = t.node;
+        sp = 0;
+        place(0, n, t.node);
     }
     __syncthreads();
     while (true) {
@@ -636,7 +659,7 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_small_build(const Task* __restr
             const int k = threadIdx.x;
             const float lo = o2f(red[6 + k]), hi = o2f(red[9 + k]);
             cb_lo[k] = lo;
-            cb_live[k] = (m > 1) && (hi - lo > 0.0f);
+            cb_live[k] = hi - lo > 0.0f;
             cb_scale[k] = cb_live[k] ? bvh_scale(lo, hi) : 0.0f;
         }
         __syncthreads();
@@ -682,50 +705,36 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_small_build(const Task* __restr
         }
         decide_block(fbins, fcounts, box, cbox, m, red_cost, red_idx, red_left, &dec);
         if (threadIdx.x == 0) {
+            // Ranges this large always split (a leaf holds at most BVH_LEAF_SIZE triangles).
+            uint32_t l = m / 2;
+            int bin_mode = 0;
+            if (dec.d.axis >= 0 && dec.left > 0 && dec.left < m) {
+                l = dec.left;
+                bin_mode = 1;
+            }
+            left = l;
+            by_bin = bin_mode;
+            axis = dec.d.axis;
+            split = dec.d.split;
+            const uint32_t ids = atomicAdd(&state[S_NODES], 2u);
             BinaryNode out;
             out.box = box;
-            live_leaf = dec.d.leaf;
-            if (dec.d.leaf) {
-                out.first = t.begin + b0;
-                out.count = m;
-                out.left = out.right = 0;
-                nodes[cur_node] = out;
+            out.left = ids;
+            out.right = ids + 1;
+            out.first = out.count = 0;
+            nodes[cur_node] = out;
+            // Smaller child on top, so it is built first.
+            const uint32_t mid = b0 + l;
+            if (l <= m - l) {
+                place(mid, e0, ids + 1);
+                place(b0, mid, ids);
             } else {
-                uint32_t l = m / 2;
-                int bin_mode = 0;
-                if (dec.d.axis >= 0 && dec.left > 0 && dec.left < m) {
-                    l = dec.left;
-                    bin_mode = 1;
-                }
-                left = l;
-                by_bin = bin_mode;
-                axis = dec.d.axis;
-                split = dec.d.split;
-                const uint32_t ids = atomicAdd(&state[S_NODES], 2u);
-                out.left = ids;
-                out.right = ids + 1;
-                out.first = 0;
-                out.count = 0;
-                nodes[cur_node] = out;
-                // Smaller child on top, so it is built first.
-                const uint32_t lb0 = b0, le0 = b0 + l, rb0 = b0 + l, re0 = e0;
-                const bool left_smaller = l <= m - l;
-                if (sp + 2 > SMALL_STACK) {
-                    atomicOr(&state[S_OVERFLOW], 16u);
-                } else {
-                    stack_b[sp] = left_smaller ? rb0 : lb0;
-                    stack_e[sp] = left_smaller ? re0 : le0;
-                    stack_n[sp] = left_smaller ? ids + 1 : ids;
-                    ++sp;
-                    stack_b[sp] = left_smaller ? lb0 : rb0;
-                    stack_e[sp] = left_smaller ? le0 : re0;
-                    stack_n[sp] = left_smaller ? ids : ids + 1;
-                    ++sp;
-                }
+                place(b0, mid, ids);
+                place(mid, e0, ids + 1);
             }
         }
         __syncthreads();
-        if (live_leaf || !by_bin) continue;  // leaves and index splits keep the order
+        if (!by_bin) continue;  // index splits keep the order
 
         // Stable partition of [b0, e0) by bin.
         const uint32_t per = (m + BUILD_BLOCK - 1) / BUILD_BLOCK;
@@ -754,6 +763,164 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_small_build(const Task* __restr
         __syncthreads();
     }
     for (uint32_t i = threadIdx.x; i < n; i += BUILD_BLOCK) order[t.begin + i] = ord[i];
+}
+
+// One wave builds the whole subtree of a range of at most WAVE_TASK
+// triangles, a triangle a lane, all ranges of a level at once: a lane folds
+// its own range's bounds, then prices, on each axis, the split after its own
+// triangle's bin, and the range takes the first of the lowest cost. Bins that
+// hold no triangle need no lane: the split after one is the split after the
+// last occupied bin below it, which the sequential sweep meets first. A level
+// loops over the longest range's lanes with shuffles; the triangles then move
+// to their side's lanes, so a range is always a run of lanes and no level
+// reads memory. Every range that is split has parts smaller than itself, so
+// at most WAVE_TASK levels follow. Bound by the loops' shuffles: 1.7 ms for a
+// million triangles, after 0.7 ms of k_small_build.
+__global__ __launch_bounds__(BUILD_BLOCK) void k_wave_build(const uint32_t* __restrict__ list, PrimArrays p,
+                                                            uint32_t* order, BinaryNode* nodes, uint32_t* state) {
+    const uint32_t lane = threadIdx.x & 63;
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+    const uint32_t tasks = state[S_WAVE];
+    const uint32_t waves = gridDim.x * (BUILD_BLOCK / 64);
+    for (uint32_t w = blockIdx.x * (BUILD_BLOCK / 64) + threadIdx.x / 64; w < tasks; w += waves) {
+        uint32_t node = list[w];
+        const uint32_t begin = nodes[node].first, total = nodes[node].count;
+        const bool in = lane < total;
+        uint32_t id = in ? order[begin + lane] : 0u;
+        Box3 b = Box3::empty();
+        float c[3] = {0.0f, 0.0f, 0.0f};
+        if (in) {
+            for (int k = 0; k < 3; ++k) {
+                b.lo[k] = p.lo[k][id];
+                b.hi[k] = p.hi[k][id];
+                c[k] = p.c[k][id];
+            }
+        }
+        // This lane's range: lanes [first, first + m); m = 0 once it is a leaf.
+        uint32_t first = in ? 0u : lane, m = in ? total : 0u;
+        while (__ballot(m > 0) != 0) {
+            // Past its range's end a lane reads itself, which changes no bound.
+            Box3 box = b, cbox;
+            for (int k = 0; k < 3; ++k) cbox.lo[k] = cbox.hi[k] = c[k];
+            for (uint32_t j = 0; __ballot(j < m) != 0; ++j) {
+                const int src = int(j < m ? first + j : lane);
+                for (int k = 0; k < 3; ++k) {
+                    box.lo[k] = fminf(box.lo[k], __shfl(b.lo[k], src));
+                    box.hi[k] = fmaxf(box.hi[k], __shfl(b.hi[k], src));
+                    const float cj = __shfl(c[k], src);
+                    cbox.lo[k] = fminf(cbox.lo[k], cj);
+                    cbox.hi[k] = fmaxf(cbox.hi[k], cj);
+                }
+            }
+            int bin[3];
+            bool live[3];
+            for (int k = 0; k < 3; ++k) {
+                live[k] = m > 1 && cbox.hi[k] - cbox.lo[k] > 0.0f;
+                bin[k] = live[k] ? bvh_bin(c[k], cbox.lo[k], bvh_scale(cbox.lo[k], cbox.hi[k])) : 0;
+            }
+            const int bins = bin[0] | bin[1] << 8 | bin[2] << 16;
+            Box3 lacc[3], racc[3];
+            uint32_t lcnt[3];
+            for (int a = 0; a < 3; ++a) {
+                lacc[a] = b;
+                racc[a] = Box3::empty();
+                lcnt[a] = 0;
+            }
+            for (uint32_t j = 0; __ballot(j < m) != 0; ++j) {
+                const int src = int(j < m ? first + j : lane);
+                Box3 o;
+                for (int k = 0; k < 3; ++k) {
+                    o.lo[k] = __shfl(b.lo[k], src);
+                    o.hi[k] = __shfl(b.hi[k], src);
+                }
+                const int ob = __shfl(bins, src);
+                for (int a = 0; a < 3; ++a) {
+                    const bool l = ((ob >> (8 * a)) & 255) <= bin[a];
+                    lcnt[a] += l && j < m;
+                    for (int k = 0; k < 3; ++k) {
+                        lacc[a].lo[k] = fminf(lacc[a].lo[k], l ? o.lo[k] : INFINITY);
+                        lacc[a].hi[k] = fmaxf(lacc[a].hi[k], l ? o.hi[k] : -INFINITY);
+                        racc[a].lo[k] = fminf(racc[a].lo[k], l ? INFINITY : o.lo[k]);
+                        racc[a].hi[k] = fmaxf(racc[a].hi[k], l ? -INFINITY : o.hi[k]);
+                    }
+                }
+            }
+            float own_cost = INFINITY;
+            uint32_t own_at = 0xffffffffu;  // axis, bin, triangles on the left
+            for (int a = 0; a < 3; ++a) {
+                const uint32_t rcnt = m - lcnt[a];
+                const float cost = lacc[a].area() * float(lcnt[a]) + racc[a].area() * float(rcnt);
+                if (live[a] && rcnt != 0 && cost < own_cost) {
+                    own_cost = cost;
+                    own_at = uint32_t(a) << 16 | uint32_t(bin[a]) << 8 | lcnt[a];
+                }
+            }
+            float best = own_cost;
+            uint32_t at = own_at;
+            for (uint32_t j = 0; __ballot(j < m) != 0; ++j) {
+                const int src = int(j < m ? first + j : lane);
+                const float oc = __shfl(own_cost, src);
+                const uint32_t oa = __shfl(own_at, src);
+                if (oc < best || (oc == best && oa < at)) {
+                    best = oc;
+                    at = oa;
+                }
+            }
+
+            // bvh_decide's choice, and the children or the leaf.
+            const float parent_area = box.area();
+            const float split_cost = BVH_NODE_COST + (parent_area > 0.0f ? best / parent_area : 0.0f);
+            const bool binned = at != 0xffffffffu;
+            const bool leaf = m <= 1 || (m <= BVH_LEAF_SIZE && (!binned || float(m) <= split_cost));
+            const bool splits = m > 0 && !leaf;
+            const uint64_t leaders = __ballot(splits && lane == first);
+            uint32_t base = 0;
+            if (leaders != 0) {
+                const int l0 = __ffsll(static_cast<unsigned long long>(leaders)) - 1;
+                if (lane == uint32_t(l0)) base = atomicAdd(&state[S_NODES], 2u * uint32_t(__popcll(leaders)));
+                base = __shfl(base, l0);
+            }
+            const uint32_t ids = base + 2u * uint32_t(__popcll(leaders & ((uint64_t(1) << first) - 1)));
+            if (m > 0 && lane == first) {
+                BinaryNode out;
+                out.box = box;
+                out.left = leaf ? 0u : ids;
+                out.right = leaf ? 0u : ids + 1;
+                out.first = leaf ? begin + first : 0u;
+                out.count = leaf ? m : 0u;
+                nodes[node] = out;
+            }
+
+            // Stable partition: every triangle to its place among the lanes.
+            const uint32_t l = binned ? at & 255u : m / 2;
+            const uint32_t bin_axis = at >> 16;
+            const int my_bin = bin_axis == 0 ? bin[0] : (bin_axis == 1 ? bin[1] : bin[2]);
+            const bool left = binned ? my_bin <= int((at >> 8) & 255u) : lane - first < l;
+            const uint64_t before = __ballot(splits && left) & below & ~((uint64_t(1) << first) - 1);
+            const uint32_t lefts = uint32_t(__popcll(before));
+            const uint32_t to = !splits ? lane : first + (left ? lefts : l + (lane - first - lefts));
+            const auto move = [&](uint32_t v) {
+                return uint32_t(__builtin_amdgcn_ds_permute(int(to * 4), int(v)));
+            };
+            id = move(id);
+            for (int k = 0; k < 3; ++k) {
+                b.lo[k] = __uint_as_float(move(__float_as_uint(b.lo[k])));
+                b.hi[k] = __uint_as_float(move(__float_as_uint(b.hi[k])));
+                c[k] = __uint_as_float(move(__float_as_uint(c[k])));
+            }
+            if (!splits) {
+                m = 0;
+            } else if (lane - first < l) {
+                node = ids;
+                m = l;
+            } else {
+                node = ids + 1;
+                first += l;
+                m -= l;
+            }
+        }
+        if (in) order[begin + lane] = id;
+    }
 }
 
 // --- the collapse to wide nodes, on the device ----------------------------------
@@ -1125,7 +1292,8 @@ bool build_bvh_device(const std::vector<WorldTriangle>& input, uint32_t max_stac
         bool keep = false;
         ~Outputs() {
             if (keep) return;
-            for (void* p : {static_cast<void*>(d->tris), static_cast<void*>(d->nodes), static_cast<void*>(d->nodes8)})
+            for (void* p : {static_cast<void*>(d->tris), static_cast<void*>(d->nodes), static_cast<void*>(d->nodes8),
+                            static_cast<void*>(d->full)})
                 if (p) (void)hipFree(p);
             *d = DeviceBvh{};
         }
@@ -1236,10 +1404,14 @@ bool build_bvh_device(const std::vector<WorldTriangle>& input, uint32_t max_stac
         BUILD_CHECK(hipGetLastError());
     }
 
-    // Subtrees, one workgroup each.
+    // Subtrees, one workgroup each, then one wave each; the waves' list lies
+    // in the scatter's second order, which nothing reads any more (its ranges
+    // are disjoint, so it has at most n entries).
     if (st[S_SMALL] > 0) {
         hipLaunchKernelGGL(k_small_build, dim3(st[S_SMALL]), dim3(BUILD_BLOCK), 0, nullptr, small, state + S_SMALL, p,
-                           order, d_nodes, state);
+                           order, d_nodes, order_tmp, n, state);
+        hipLaunchKernelGGL(k_wave_build, dim3(std::min<uint32_t>(blocks_for(n), 2048)), dim3(BUILD_BLOCK), 0, nullptr,
+                           order_tmp, p, order, d_nodes, state);
         BUILD_CHECK(hipGetLastError());
     }
     BUILD_CHECK(hipMemcpy(st, state, sizeof(st), hipMemcpyDeviceToHost));
@@ -1265,37 +1437,26 @@ bool build_bvh_device(const std::vector<WorldTriangle>& input, uint32_t max_stac
         if (deep) *error = "BVH too deep for the traversal stack (depth " + std::to_string(depth4) + ")";
         return false;
     }
-    BvhNode4* full4 = s.get<BvhNode4>(count4);
-    BvhNode4Q* quant4 = nullptr;
-    BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&quant4), sizeof(BvhNode4Q) * count4));
-    dev->nodes = quant4;
-    if (!full4) {
-        *error = "device BVH build: out of device memory";
-        return false;
-    }
+    BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&dev->full), sizeof(BvhNode4) * count4));
+    BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&dev->nodes), sizeof(BvhNode4Q) * count4));
+    dev->node_count = count4;
     const uint32_t grid4 = std::min<uint32_t>(blocks_for(count4), 2048);
     hipLaunchKernelGGL(k_collapse_write4, dim3(grid4), dim3(BUILD_BLOCK), 0, nullptr, d_nodes, wide4, idx4, state,
-                       state + S_MAX_ABS, full4, quant4);
+                       state + S_MAX_ABS, dev->full, dev->nodes);
     BUILD_CHECK(hipGetLastError());
-    out->nodes.resize(count4);
-    BUILD_CHECK(hipMemcpy(out->nodes.data(), full4, sizeof(BvhNode4) * count4, hipMemcpyDeviceToHost));
     out->max_depth = depth4;
 
     WideTmp<8>* wide8 = nullptr;
     uint32_t* idx8 = nullptr;
     uint32_t depth8 = 0, count8 = 0;
-    out->nodes8.clear();
     out->max_depth8 = 0;
     if (collapse_device<8>(d_nodes, n, state, max_stack / 7, s, &wide8, &idx8, &depth8, &count8, &deep, error)) {
-        BvhNode8Q* quant8 = nullptr;
-        BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&quant8), sizeof(BvhNode8Q) * count8));
-        dev->nodes8 = quant8;
+        BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&dev->nodes8), sizeof(BvhNode8Q) * count8));
+        dev->node8_count = count8;
         const uint32_t grid8 = std::min<uint32_t>(blocks_for(count8), 2048);
         hipLaunchKernelGGL(k_collapse_write8, dim3(grid8), dim3(BUILD_BLOCK), 0, nullptr, d_nodes, wide8, idx8, state,
-                           state + S_MAX_ABS, quant8);
+                           state + S_MAX_ABS, dev->nodes8);
         BUILD_CHECK(hipGetLastError());
-        out->nodes8.resize(count8);
-        BUILD_CHECK(hipMemcpy(out->nodes8.data(), quant8, sizeof(BvhNode8Q) * count8, hipMemcpyDeviceToHost));
         out->max_depth8 = depth8;
     } else if (!deep) {
         return false;

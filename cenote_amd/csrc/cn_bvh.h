@@ -62,14 +62,16 @@ struct DeviceBvh {
     BvhTriangle* tris = nullptr;
     BvhNode4Q* nodes = nullptr;
     BvhNode8Q* nodes8 = nullptr;
+    BvhNode4* full = nullptr;  // the full-precision nodes, for read-back
+    uint32_t node_count = 0, node8_count = 0;
 };
 
 // The same trees built entirely on the device (cn_build.hip): top levels by
 // device-wide binning with every split decided on the device, subtrees of
-// <= 2048 triangles by one workgroup each, the collapse to 4- and 8-wide
-// nodes and their quantization on the device. `out` receives host copies of
-// the full-precision 4-wide nodes and the quantized 8-wide nodes (for
-// read-back); the traversal's arrays stay on the device in `*dev`.
+// <= 2048 triangles by one workgroup each and of <= 64 by one wave each, the
+// collapse to 4- and 8-wide
+// nodes and their quantization on the device, where the trees stay (`*dev`);
+// `out` receives the depths and the build time.
 bool build_bvh_device(const std::vector<WorldTriangle>& input, uint32_t max_stack, Bvh4* out, DeviceBvh* dev,
                       std::string* error);
 

@@ -289,14 +289,15 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
         quantize_bvh4(bvh.nodes.data(), bvh.nodes.size(), quantized.data());
         CN_HIP(scene->nodes.upload(quantized.data(), quantized.size()));
         if (!bvh.nodes8.empty()) CN_HIP(scene->nodes8.upload(bvh.nodes8.data(), bvh.nodes8.size()));
+        CN_HIP(scene->full_nodes.upload(bvh.nodes.data(), bvh.nodes.size()));
     } else {
-        // Built, collapsed and quantized on the device; the host keeps
-        // copies only for read-back (cn_scene_bvh, cn_scene_bvh8).
+        // Built, collapsed and quantized on the device, and kept there.
         DeviceBvh dev;
         if (!build_bvh_device(world, STACK_MAX, &bvh, &dev, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
         scene->tris.adopt(dev.tris, world.size());
-        scene->nodes.adopt(dev.nodes, bvh.nodes.size());
-        if (dev.nodes8) scene->nodes8.adopt(dev.nodes8, bvh.nodes8.size());
+        scene->nodes.adopt(dev.nodes, dev.node_count);
+        scene->full_nodes.adopt(dev.full, dev.node_count);
+        if (dev.nodes8) scene->nodes8.adopt(dev.nodes8, dev.node8_count);
     }
     CN_HIP(scene->pnodes.alloc(scene->nodes.count));
     if (!decode_packet_nodes(scene->nodes.ptr, uint32_t(scene->nodes.count), scene->pnodes.ptr, &error))
@@ -321,17 +322,15 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
     cn_scene_info& info = scene->info;
     info.instance_count = desc->instance_count;
     info.triangle_count = uint32_t(world.size());
-    info.bvh_node_count = uint32_t(bvh.nodes.size());
-    scene->host_nodes = std::move(bvh.nodes);
+    info.bvh_node_count = uint32_t(scene->nodes.count);
     info.bvh_width = 4;
     info.bvh_node_bytes = sizeof(BvhNode4Q);
     info.bvh_triangle_bytes = sizeof(BvhTriangle);
     info.bvh_max_depth = bvh.max_depth;
     info.bvh_builder = desc->bvh_builder;
     info.bvh_build_seconds = bvh.build_seconds;
-    info.bvh8_node_count = uint32_t(bvh.nodes8.size());
-    info.bvh8_max_depth = bvh.nodes8.empty() ? 0u : bvh.max_depth8;
-    scene->host_nodes8 = std::move(bvh.nodes8);
+    info.bvh8_node_count = uint32_t(scene->nodes8.count);
+    info.bvh8_max_depth = scene->nodes8.count == 0 ? 0u : bvh.max_depth8;
     return CN_OK;
 }
 
@@ -493,11 +492,11 @@ int cn_scene_bvh(cn_scene* scene, void* nodes, uint32_t node_capacity, uint32_t*
                  uint32_t triangle_capacity, uint32_t* triangle_count) {
     if (!scene) return fail(CN_E_INVALID, "cn_scene_bvh: null scene");
     CN_HIP(hipSetDevice(scene->ctx->device));
-    if (node_count) *node_count = uint32_t(scene->host_nodes.size());
+    if (node_count) *node_count = uint32_t(scene->full_nodes.count);
     if (triangle_count) *triangle_count = uint32_t(scene->tris.count);
     if (nodes) {
-        if (node_capacity < scene->host_nodes.size()) return fail(CN_E_INVALID, "node buffer too small");
-        std::memcpy(nodes, scene->host_nodes.data(), scene->host_nodes.size() * sizeof(BvhNode4));
+        if (node_capacity < scene->full_nodes.count) return fail(CN_E_INVALID, "node buffer too small");
+        CN_HIP(hipMemcpy(nodes, scene->full_nodes.ptr, scene->full_nodes.count * sizeof(BvhNode4), hipMemcpyDeviceToHost));
     }
     if (triangles) {
         if (triangle_capacity < scene->tris.count) return fail(CN_E_INVALID, "triangle buffer too small");
@@ -508,10 +507,11 @@ int cn_scene_bvh(cn_scene* scene, void* nodes, uint32_t node_capacity, uint32_t*
 
 int cn_scene_bvh8(cn_scene* scene, void* nodes, uint32_t node_capacity, uint32_t* node_count) {
     if (!scene) return fail(CN_E_INVALID, "cn_scene_bvh8: null scene");
-    if (node_count) *node_count = uint32_t(scene->host_nodes8.size());
+    if (node_count) *node_count = uint32_t(scene->nodes8.count);
     if (nodes) {
-        if (node_capacity < scene->host_nodes8.size()) return fail(CN_E_INVALID, "node buffer too small");
-        std::memcpy(nodes, scene->host_nodes8.data(), scene->host_nodes8.size() * sizeof(BvhNode8Q));
+        if (node_capacity < scene->nodes8.count) return fail(CN_E_INVALID, "node buffer too small");
+        CN_HIP(hipSetDevice(scene->ctx->device));
+        CN_HIP(hipMemcpy(nodes, scene->nodes8.ptr, scene->nodes8.count * sizeof(BvhNode8Q), hipMemcpyDeviceToHost));
     }
     return CN_OK;
 }
