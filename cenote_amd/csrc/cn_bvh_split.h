@@ -14,12 +14,17 @@
 namespace cn {
 
 constexpr int BVH_BINS = 32;
-constexpr uint32_t BVH_LEAF_SIZE = 8;
-// A node step costs about two triangle tests in the traversal (four boxes,
-// the child ordering and a stack operation against one watertight test):
-// the SAH's traversal term, measured best of 1, 1.5 and 2 on the 2M-triangle
-// benchmark scene.
-constexpr float BVH_NODE_COST = 2.0f;
+// The SAH's traversal term and the largest leaf, for the voted walk of the
+// trace kernel: a triangle step of a wave costs about as much as a node step
+// (90 to 150 instructions against 140, and both end the vote's turn), and its
+// lanes wait on it, so small leaves pay. Trace ms per frame at node cost 2,
+// 1.4, 1, 0.7, 0.5 (2M triangles from inside): 26.0, 25.0, 24.4, 24.2, 24.0;
+// from outside 11.7, 11.3, 11.0, 11.0, 11.0; the Cornell box, whose 36
+// triangles make a few leaves, 0.605 and then 0.465. Leaves of 8, 4, 3 and 2
+// measured within 2% of one another below cost 1; 4 keeps the tree smaller
+// than 2.
+constexpr uint32_t BVH_LEAF_SIZE = 4;
+constexpr float BVH_NODE_COST = 0.7f;
 
 struct Box3 {
     float lo[3], hi[3];
@@ -59,7 +64,7 @@ struct SplitDecision {
     int split;  // bins 0..split go left
 };
 
-// Binned SAH over the three axes (32 bins; leaves of <= 8 triangles when a
+// Binned SAH over the three axes (32 bins; leaves of <= 4 triangles when a
 // leaf is no costlier than the best split, a triangle test costing 1 and a
 // node step BVH_NODE_COST). `bins`/`counts` hold the
 // range's per-axis bins; axes whose centroid extent is not positive are
