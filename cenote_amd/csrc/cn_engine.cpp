@@ -345,6 +345,16 @@ uint32_t samples_per_wave(const cn_renderer* r, uint32_t pixels, uint32_t wanted
     return std::min({wanted, fit, 65535u});
 }
 
+int film_read_back(cn_film* f, float divisor, float* beauty, float* albedo, float* normal, float* depth) {
+    const size_t n = size_t(f->width) * f->height;
+    auto array = [&](const void* src, float* out, size_t lanes) {
+        return ReadArray{static_cast<const float*>(src), out, n * lanes, divisor};
+    };
+    const ReadArray arrays[4] = {array(f->beauty_sum.ptr, beauty, 4), array(f->albedo_sum.ptr, albedo, 4),
+                                 array(f->normal_sum.ptr, normal, 4), array(f->depth_sum.ptr, depth, 1)};
+    return read_back(f->ctx->device, f->ctx->readback, arrays, 4);
+}
+
 int film_job(cn_renderer* r, cn_scene* s, cn_film* f, const cn_camera& camera, uint32_t samples, HostJob* job) {
     job->scene = s;
     job->width = f->width;
@@ -587,23 +597,12 @@ int cn_trace_aov(cn_renderer* r, cn_scene* s, float* radiance, float* albedo, fl
     CN_HIP(hipStreamSynchronize(r->stream));
     // The slots hold the view in band order (band_pixel); the images are
     // row-major.
-    auto fetch = [&](void* out, const void* slots, size_t bytes) -> int {
-        std::vector<unsigned char> tmp(pixels * bytes);
-        CN_HIP(hipMemcpy(tmp.data(), slots, tmp.size(), hipMemcpyDeviceToHost));
-        unsigned char* dst = static_cast<unsigned char*>(out);
-        for (uint32_t i = 0; i < pixels; ++i)
-            std::memcpy(dst + size_t(band_pixel(i, width, height)) * bytes, tmp.data() + size_t(i) * bytes, bytes);
-        return CN_OK;
+    auto image = [&](const void* slots, float* out, uint32_t lanes) {
+        return ReadArray{static_cast<const float*>(slots), out, pixels * lanes, 1.0f, lanes, width, height};
     };
-    if (radiance)
-        if (int e = fetch(radiance, r->radiance.ptr, 16)) return e;
-    if (albedo)
-        if (int e = fetch(albedo, r->albedo.ptr, 16)) return e;
-    if (normal)
-        if (int e = fetch(normal, r->normal.ptr, 16)) return e;
-    if (depth)
-        if (int e = fetch(depth, r->depth.ptr, 4)) return e;
-    return CN_OK;
+    const ReadArray images[4] = {image(r->radiance.ptr, radiance, 4), image(r->albedo.ptr, albedo, 4),
+                                 image(r->normal.ptr, normal, 4), image(r->depth.ptr, depth, 1)};
+    return read_back(r->ctx->device, r->ctx->readback, images, 4);
 }
 
 int cn_trace(cn_renderer* r, cn_scene* s, float* radiance, uint32_t width, uint32_t height, uint32_t sample) {
@@ -744,30 +743,16 @@ int cn_film_sums(cn_film* f, float* beauty, float* albedo, float* normal, float*
     if (!f) return fail(CN_E_INVALID, "cn_film_sums: null film");
     CN_HIP(hipSetDevice(f->ctx->device));
     CN_HIP(hipDeviceSynchronize());
-    const size_t n = size_t(f->width) * f->height;
-    if (beauty) CN_HIP(hipMemcpy(beauty, f->beauty_sum.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (albedo) CN_HIP(hipMemcpy(albedo, f->albedo_sum.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (normal) CN_HIP(hipMemcpy(normal, f->normal_sum.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (depth) CN_HIP(hipMemcpy(depth, f->depth_sum.ptr, n * 4, hipMemcpyDeviceToHost));
-    return CN_OK;
+    return film_read_back(f, 1.0f, beauty, albedo, normal, depth);
 }
 
 int cn_film_averages(cn_film* f, float* beauty, float* albedo, float* normal, float* depth) {
     if (!f) return fail(CN_E_INVALID, "cn_film_averages: null film");
     if (f->samples == 0) return fail(CN_E_INVALID, "averaging an empty film");
-    const size_t n = size_t(f->width) * f->height;
-    if (int e = cn_film_sums(f, beauty, albedo, normal, depth)) return e;
+    CN_HIP(hipSetDevice(f->ctx->device));
+    CN_HIP(hipDeviceSynchronize());
     // render/film.rs:194-197: sum / samples on the host.
-    const float samples = float(f->samples);
-    auto divide = [&](float* a, size_t count) {
-        if (a)
-            for (size_t i = 0; i < count; ++i) a[i] = a[i] / samples;
-    };
-    divide(beauty, 4 * n);
-    divide(albedo, 4 * n);
-    divide(normal, 4 * n);
-    divide(depth, n);
-    return CN_OK;
+    return film_read_back(f, float(f->samples), beauty, albedo, normal, depth);
 }
 
 int cn_film_set_sample(cn_film* f, const float* beauty, const float* albedo, const float* normal,
@@ -837,11 +822,12 @@ int cn_resolve(cn_renderer* r, cn_film* f, float* beauty, float* albedo, float* 
                f->out_normal.ptr, f->normal_sum.ptr, f->out_depth.ptr, f->depth_sum.ptr};
     CN_HIP(launch_resolve(r->stream, v, uint32_t(n), float(f->samples)));
     CN_HIP(hipStreamSynchronize(r->stream));
-    if (beauty) CN_HIP(hipMemcpy(beauty, f->out_beauty.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (albedo) CN_HIP(hipMemcpy(albedo, f->out_albedo.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (normal) CN_HIP(hipMemcpy(normal, f->out_normal.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (depth) CN_HIP(hipMemcpy(depth, f->out_depth.ptr, n * 4, hipMemcpyDeviceToHost));
-    return CN_OK;
+    auto array = [&](const void* src, float* out, size_t lanes) {
+        return ReadArray{static_cast<const float*>(src), out, n * lanes};
+    };
+    const ReadArray arrays[4] = {array(f->out_beauty.ptr, beauty, 4), array(f->out_albedo.ptr, albedo, 4),
+                                 array(f->out_normal.ptr, normal, 4), array(f->out_depth.ptr, depth, 1)};
+    return read_back(r->ctx->device, r->ctx->readback, arrays, 4);
 }
 
 int cn_sample_sequence(cn_context* ctx, uint32_t pixel, uint32_t dimension, uint32_t count, float* points2d,

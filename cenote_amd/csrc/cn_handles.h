@@ -14,6 +14,7 @@
 #include "../../include/cenote_hip.h"
 #include "cn_launch.h"
 #include "cn_prep.h"
+#include "cn_readback.h"
 #include "cn_records.h"
 
 namespace cn {
@@ -101,6 +102,7 @@ struct cn_context {
     uint32_t compute_units = 0;
     std::string name;
     cn::DevBuf<float> tables;  // the BSDF tables, shared by every scene
+    cn::Readback readback;     // staging of results on their way to the host
 };
 
 struct cn_scene {
@@ -188,6 +190,10 @@ int enqueue_wave(cn_renderer* r, std::vector<HostJob> jobs, bool aov, const Wave
 // A film job for `samples` more samples of `camera` on `s`, continuing at
 // the film's sample count.
 int film_job(cn_renderer* r, cn_scene* s, cn_film* f, const cn_camera& camera, uint32_t samples, HostJob* job);
+
+// The film's sums over `divisor` into host arrays (any may be null); what
+// folds into the film must have finished.
+int film_read_back(cn_film* f, float divisor, float* beauty, float* albedo, float* normal, float* depth);
 
 // Samples of a `pixels`-pixel view that fill one wave of the renderer's pool.
 uint32_t samples_per_wave(const cn_renderer* r, uint32_t pixels, uint32_t wanted);

@@ -487,21 +487,8 @@ int cn_server_result(cn_server* sv, uint64_t id, float* beauty, float* albedo, f
     if (!q.film) return fail(CN_E_INVALID, "request %llu's result was already taken", (unsigned long long)id);
     CN_HIP(hipSetDevice(sv->r->ctx->device));
     // Every wave that touched this film has retired (its event completed).
-    const size_t n = size_t(q.desc.width) * q.desc.height;
     cn_film* f = q.film;
-    if (beauty) CN_HIP(hipMemcpy(beauty, f->beauty_sum.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (albedo) CN_HIP(hipMemcpy(albedo, f->albedo_sum.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (normal) CN_HIP(hipMemcpy(normal, f->normal_sum.ptr, n * 16, hipMemcpyDeviceToHost));
-    if (depth) CN_HIP(hipMemcpy(depth, f->depth_sum.ptr, n * 4, hipMemcpyDeviceToHost));
-    const float samples = float(q.completed);
-    auto divide = [&](float* a, size_t count) {
-        if (a)
-            for (size_t i = 0; i < count; ++i) a[i] = a[i] / samples;
-    };
-    divide(beauty, 4 * n);
-    divide(albedo, 4 * n);
-    divide(normal, 4 * n);
-    divide(depth, n);
+    if (int e = film_read_back(f, float(q.completed), beauty, albedo, normal, depth)) return e;
     sv->spare.emplace(std::make_pair(q.desc.width, q.desc.height), f);
     sv->spare_bytes += q.bytes;
     q.film = nullptr;
