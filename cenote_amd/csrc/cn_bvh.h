@@ -66,13 +66,24 @@ struct DeviceBvh {
     uint32_t node_count = 0, node8_count = 0;
 };
 
+// A scene's triangles as the device builder reads them: instance i's are the
+// mesh triangles from its record's triangle_base on, numbered
+// first[i] .. first[i + 1] - 1 in the scene.
+struct DeviceTriangles {
+    const MeshTriangle* mesh_tris;    // device
+    const InstanceRecord* instances;  // device
+    const uint32_t* flags;            // host, one word per instance
+    const size_t* first;              // host, instance_count + 1
+    uint32_t instance_count;
+};
+
 // The same trees built entirely on the device (cn_build.hip): top levels by
 // device-wide binning with every split decided on the device, subtrees of
 // <= 2048 triangles by one workgroup each and of <= 64 by one wave each, the
 // collapse to 4- and 8-wide
 // nodes and their quantization on the device, where the trees stay (`*dev`);
 // `out` receives the depths and the build time.
-bool build_bvh_device(const std::vector<WorldTriangle>& input, uint32_t max_stack, Bvh4* out, DeviceBvh* dev,
+bool build_bvh_device(const DeviceTriangles& input, uint32_t max_stack, Bvh4* out, DeviceBvh* dev,
                       std::string* error);
 
 // Rewrites, on the device, the flags word (v2.w) of every leaf-order

@@ -264,8 +264,14 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
     std::vector<cn_material> materials;
     std::vector<uint32_t> tri_flags;
     std::vector<EmissiveTriangle> emitters;
-    std::vector<WorldTriangle> world;
-    if (int e = prep_instances(desc, pool, &records, &materials, &tri_flags, &emitters, &world)) return e;
+    std::vector<WorldTriangle> world;  // for the host builder
+    const bool host_built = desc->bvh_builder == CN_BVH_HOST;
+    if (int e = prep_instances(desc, pool, &records, &materials, &tri_flags, &emitters, host_built ? &world : nullptr))
+        return e;
+    std::vector<size_t> first(size_t(desc->instance_count) + 1, 0);  // each instance's first triangle
+    for (uint32_t i = 0; i < desc->instance_count; ++i)
+        first[i + 1] = first[i] + desc->meshes[desc->instances[i].mesh].triangle_count;
+    const size_t triangle_count = first.back();
 
     scene->ctx = ctx;
     scene->camera = desc->camera;
@@ -280,9 +286,13 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
         for (size_t k = 0; k < 3 * size_t(mesh.triangle_count); ++k) out[k] = base + mesh.indices[k];
     }
 
+    CN_HIP(scene->instances.upload(records.data(), records.size()));
+    CN_HIP(scene->mesh_tris.alloc(pool.triangles));
+    CN_HIP(build_mesh_triangles(positions.data(), normals.data(), pool.vertices, indices.data(), pool.triangles,
+                                scene->mesh_tris.ptr));
     Bvh4 bvh;
     std::string error;
-    if (desc->bvh_builder == CN_BVH_HOST) {
+    if (host_built) {
         if (!build_bvh4(world, STACK_MAX, &bvh, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
         CN_HIP(scene->tris.upload(bvh.tris.data(), bvh.tris.size()));
         std::vector<BvhNode4Q> quantized(bvh.nodes.size());
@@ -293,8 +303,10 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
     } else {
         // Built, collapsed and quantized on the device, and kept there.
         DeviceBvh dev;
-        if (!build_bvh_device(world, STACK_MAX, &bvh, &dev, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
-        scene->tris.adopt(dev.tris, world.size());
+        const DeviceTriangles input{scene->mesh_tris.ptr, scene->instances.ptr, tri_flags.data(), first.data(),
+                                    desc->instance_count};
+        if (!build_bvh_device(input, STACK_MAX, &bvh, &dev, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
+        scene->tris.adopt(dev.tris, triangle_count);
         scene->nodes.adopt(dev.nodes, dev.node_count);
         scene->full_nodes.adopt(dev.full, dev.node_count);
         if (dev.nodes8) scene->nodes8.adopt(dev.nodes8, dev.node8_count);
@@ -302,11 +314,7 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
     CN_HIP(scene->pnodes.alloc(scene->nodes.count));
     if (!decode_packet_nodes(scene->nodes.ptr, uint32_t(scene->nodes.count), scene->pnodes.ptr, &error))
         return fail(CN_E_SCENE, "%s", error.c_str());
-    CN_HIP(scene->instances.upload(records.data(), records.size()));
     CN_HIP(scene->materials.upload(materials.data(), materials.size()));
-    CN_HIP(scene->mesh_tris.alloc(pool.triangles));
-    CN_HIP(build_mesh_triangles(positions.data(), normals.data(), pool.vertices, indices.data(), pool.triangles,
-                                scene->mesh_tris.ptr));
     if (int e = install_lights(scene, std::move(emitters), desc->delta_lights, desc->delta_light_count)) return e;
     if (int e = install_environment(scene, desc->environment)) return e;
     scene->host_records = std::move(records);
@@ -321,7 +329,7 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
 
     cn_scene_info& info = scene->info;
     info.instance_count = desc->instance_count;
-    info.triangle_count = uint32_t(world.size());
+    info.triangle_count = uint32_t(triangle_count);
     info.bvh_node_count = uint32_t(scene->nodes.count);
     info.bvh_width = 4;
     info.bvh_node_bytes = sizeof(BvhNode4Q);

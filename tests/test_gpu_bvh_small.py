@@ -1,4 +1,4 @@
-"""The device builder's wave subtrees against the host builder, at the edges.
+"""The device builder against the host builder, at the edges of its steps.
 
 Ranges of at most 64 triangles are built by one wave, a triangle a lane;
 larger ones come to it through a workgroup's splits. Both builders must grow
@@ -41,6 +41,29 @@ def test_small_ranges_match_the_host_builder(ctx, kind, count):
     for builder in (_abi.BVH_HOST, _abi.BVH_DEVICE):
         scene = cn.Scene(ctx, data, bvh_builder=builder)
         trees.append((*scene.bvh(), scene.bvh8()))
+        scene.close()
+    for host, device in zip(*trees):
+        assert np.asarray(host).tobytes() == np.asarray(device).tobytes()
+
+
+@pytest.mark.parametrize("counts", [(7,), (0, 5, 0, 0, 70, 0), (1, 1, 300, 1)])
+def test_instances_reach_the_world_as_the_host_takes_them(ctx, counts):
+    data = SceneData()
+    rng = np.random.default_rng(len(counts))
+    meshes = []
+    for count in counts:
+        p = rng.uniform(-1, 1, (3 * count, 3)).astype(np.float32)
+        n = np.tile(np.array([0.0, 0.0, 1.0], np.float32), (3 * count, 1))
+        meshes.append(data.add_mesh(MeshData(p, n, np.arange(3 * count, dtype=np.uint32).reshape(-1, 3))))
+    for k, mesh in enumerate(meshes + meshes[::-1]):
+        t = np.asarray(identity(), np.float32).reshape(3, 4) + rng.normal(scale=0.3, size=(3, 4)).astype(np.float32)
+        data.add_instance(mesh, t.reshape(np.shape(identity())), Material.matte((0.1 * k, 0.5, 0.5)))
+    data.env_texels = np.ones((1, 1, 4), np.float32)
+    trees = []
+    for builder in (_abi.BVH_HOST, _abi.BVH_DEVICE):
+        scene = cn.Scene(ctx, data, bvh_builder=builder)
+        trees.append((*scene.bvh(), scene.bvh8()))
+        assert scene.info().triangle_count == 2 * sum(counts)
         scene.close()
     for host, device in zip(*trees):
         assert np.asarray(host).tobytes() == np.asarray(device).tobytes()
