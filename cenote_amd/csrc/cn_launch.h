@@ -37,8 +37,9 @@ struct LaunchShape {
     uint32_t shade_blocks;   // most blocks (of the variant's size) for shade_surface
     uint32_t light_blocks;   // blocks of 256 lanes for shade_miss
     uint32_t bvh_width;      // 4 or 8: the tree the traversal kernels walk
-    uint32_t tail_bounce;    // 0: every bounce runs as wavefront stages; b >= 1: after bounce b's
-                             // trace, one tail launch carries each live path to its end
+    uint32_t tail_bounce;    // 0: every bounce runs as wavefront stages; b >= 1: after the trace of
+                             // bounce b, or of an earlier one with few rays, one tail launch
+                             // carries each live path to its end
 };
 
 // The film's buffers (render/film.rs:66-127): one wave's sample
@@ -70,16 +71,17 @@ struct Profiler {
 // Starts a range of a wave: resets its queue counters.
 hipError_t launch_raygen(hipStream_t stream, uint32_t* counters, uint32_t counter_lines, Profiler* prof);
 
-// One bounce: trace, then shade_miss and shade_surface — or, with `tail`,
-// trace and then the tail launch that finishes every live path (its item
-// counters at `tail_claims`, zeroed with the range's other counters; its
-// grid the waves `compute_units` CUs hold at once). Bounce 0's trace
+// One bounce: trace, then shade_miss and shade_surface — or, at
+// `tail_bounce` (UINT32_MAX: never), trace and then the tail launch that
+// finishes every live path (its item counters zeroed with the range's other
+// counters; its grid the waves `compute_units` CUs hold at once). Where a
+// tail launch follows, bounces with few rays are left to it. Bounce 0's trace
 // generates the camera paths of slots [base, base + range_count) of a wave
 // whose jobs (sorted by slot base) are `jobs[0 .. job_count)`.
 hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const SceneView& s, const PathPool& p,
                          const WaveTargets& tg, uint32_t* counters, const JobRecord* jobs, uint32_t job_count,
                          uint32_t base, uint32_t range_count, uint32_t bounce, uint32_t light_sampling, int counting,
-                         bool tail, uint32_t max_bounces, uint32_t compute_units, Profiler* prof);
+                         uint32_t tail_bounce, uint32_t max_bounces, uint32_t compute_units, Profiler* prof);
 
 // Fold every job's slots into its film sums (jobs sorted by pixel base;
 // total_pixels is the sum of the jobs' view pixels).

@@ -69,6 +69,21 @@ __device__ __forceinline__ uint32_t queue_total(const uint32_t* counters, uint32
     return total;
 }
 
+// Whether the tail launch takes the paths of `bounce` (and so of every later
+// one): the bounce has no more than `hand_over` of them. The stages then
+// leave it alone, each launch returning on its first counter reads, and the
+// tail starts there instead of at its own bounce: a small bounce costs its
+// three launches about 90 us of dependent fetches whatever it holds, a path in
+// the tail some 20 us a bounce. Per pass at TAIL_PATHS 0 (never), 8192, 16384,
+// 49152: a 64 x 64 view of the Cornell box 0.345, 0.30, 0.293, 0.30 ms; a
+// 320 x 180 view of the 2M triangles, edited, 1.37, 1.19, 1.20, 1.24; the eight
+// waves of a 720p session 9.3, 8.45, 8.45, 8.8; the veiled chart 2.87, 2.77,
+// 2.77, 2.79; waves of a million paths and more unchanged.
+constexpr uint32_t TAIL_PATHS = 16384;
+__device__ __forceinline__ bool handed_over(const uint32_t* counters, uint32_t bounce, uint32_t hand_over) {
+    return bounce > 0 && queue_total(counters, bounce, Q_RAY) <= hand_over;
+}
+
 // Array position of the queue's i-th entry (i < its total).
 __device__ __forceinline__ uint32_t queue_slot(const uint32_t* counters, uint32_t bounce, Queue queue, uint32_t i,
                                                uint32_t sub_capacity) {
@@ -234,7 +249,9 @@ __device__ __forceinline__ void miss_path(const SceneView& s, const PathPool& p,
 }
 
 __global__ __launch_bounds__(BLOCK) void k_shade_miss(SceneView s, PathPool p, WaveTargets tg, uint32_t* counters,
-                                                      uint32_t base, uint32_t bounce, uint32_t light_sampling) {
+                                                      uint32_t base, uint32_t bounce, uint32_t light_sampling,
+                                                      uint32_t hand_over) {
+    if (handed_over(counters, bounce, hand_over)) return;
     const uint32_t n = queue_total(counters, bounce, Q_MISS);
     for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
         const uint32_t path = p.miss_queue[queue_slot(counters, bounce, Q_MISS, i, p.sub_capacity)];
@@ -783,7 +800,9 @@ __device__ __forceinline__ bool shade_path(const SceneView& s, const PathPool& p
 // path's own slot.
 template <uint32_t SB, bool LDS_TABLES, bool SORT>
 __global__ __launch_bounds__(SB) __attribute__((amdgpu_waves_per_eu(3))) void k_shade_surface(SceneView s, PathPool p, WaveTargets tg, uint32_t* counters,
-                                                      uint32_t base, uint32_t bounce, uint32_t light_sampling) {
+                                                      uint32_t base, uint32_t bounce, uint32_t light_sampling,
+                                                      uint32_t hand_over) {
+    if (handed_over(counters, bounce, hand_over)) return;
     const uint32_t n = queue_total(counters, bounce, Q_HIT);
     if (blockIdx.x * SB >= n) return;  // uniform per block: nothing to shade here
     const float* tables = s.tables;
@@ -902,7 +921,7 @@ __global__ __launch_bounds__(SB) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // Past the first few bounces a wave holds few live paths, and each bounce's
 // three launches last as long as the slowest of them: the deep bounces cost
 // the sum, over bounces, of the slowest path's latency. From a chosen bounce
-// on, one launch takes every path of that bounce's miss and hit queues
+// on, or from the first that is small enough (handed_over), one launch takes every path of that bounce's miss and hit queues
 // through all of its remaining bounces — shading, the next-event connection
 // traced at once, the next closest hit — with the wavefront kernels' own
 // device functions. A slot sees the same adds in the same order as in the
@@ -918,9 +937,14 @@ __global__ __launch_bounds__(SB) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // after both walks and before it shades the next hit.
 template <bool W8>
 __global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu(TAIL_WAVES))) void k_tail(
-    SceneView s, PathPool p, WaveTargets tg, uint32_t* counters, uint32_t* claims, uint32_t base, uint32_t bounce,
-    uint32_t light_sampling) {
+    SceneView s, PathPool p, WaveTargets tg, uint32_t* counters, uint32_t* claims, uint32_t base, uint32_t last_bounce,
+    uint32_t light_sampling, uint32_t hand_over) {
     __shared__ uint32_t lds_stack[STACK_LDS * TRAVERSAL_BLOCK];
+    // The stages stopped at the first bounce that was handed over. Its
+    // counters are final; those of later bounces are counted up below, so
+    // that bounces up to last_bounce are counted whoever carried them.
+    uint32_t bounce = 1;
+    while (bounce < last_bounce && !handed_over(counters, bounce, hand_over)) ++bounce;
     const uint32_t n_miss = queue_total(counters, bounce, Q_MISS);
     const uint32_t n = n_miss + queue_total(counters, bounce, Q_HIT);
     const uint32_t lanes = gridDim.x * TRAVERSAL_BLOCK;
@@ -1035,6 +1059,13 @@ __global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu
                                       : 1.0f;
                 att = __shfl(att, mate);
                 if (!helper && connect && att > 0.0f) add_pixel(tg.radiance, sh.pixel, sh.contrib * att, 0.0f);
+            if (!helper && b < last_bounce) {  // counted as the stages count; a wave's pairs are at different bounces
+                if (connect) atomicAdd(&counters[counter_index(b, Q_SHADOW, stripe)], 1u);
+                if (next) {
+                    atomicAdd(&counters[counter_index(b + 1, Q_RAY, stripe)], 1u);
+                    atomicAdd(&counters[counter_index(b + 1, best.hit() ? Q_HIT : Q_MISS, stripe)], 1u);
+                }
+            }
             if (!next) {
                 live = false;
             } else {
@@ -1358,7 +1389,9 @@ hipError_t launch_raygen(hipStream_t stream, uint32_t* counters, uint32_t counte
 hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const SceneView& s, const PathPool& p,
                          const WaveTargets& tg, uint32_t* counters, const JobRecord* jobs, uint32_t job_count,
                          uint32_t base, uint32_t range_count, uint32_t bounce, uint32_t light_sampling, int counting,
-                         bool tail, uint32_t max_bounces, uint32_t compute_units, Profiler* prof) {
+                         uint32_t tail_bounce, uint32_t max_bounces, uint32_t compute_units, Profiler* prof) {
+    const bool tail = bounce == tail_bounce;
+    const uint32_t hand_over = tail_bounce == UINT32_MAX ? 0u : TAIL_PATHS;
     const uint32_t light_grid = grid_for(range_count, shape.light_blocks);
     // Bounce b's rays and bounce b-1's shadow rays share one launch; the
     // last bounce shades terminally and leaves no shadow rays behind.
@@ -1407,17 +1440,17 @@ hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const Sce
         if (prof) prof->begin(K_TAIL);
         if (wide)
             hipLaunchKernelGGL(k_tail<true>, dim3(tail_grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg, counters,
-                               counters + tail_claim_index(max_bounces), base, bounce, light_sampling);
+                               counters + tail_claim_index(max_bounces), base, bounce, light_sampling, hand_over);
         else
             hipLaunchKernelGGL(k_tail<false>, dim3(tail_grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg, counters,
-                               counters + tail_claim_index(max_bounces), base, bounce, light_sampling);
+                               counters + tail_claim_index(max_bounces), base, bounce, light_sampling, hand_over);
         if (prof) prof->end(K_TAIL);
         return hipGetLastError();
     }
     if (bounce > 0) {  // bounce 0's misses were shaded by the trace launch
         if (prof) prof->begin(K_SHADE_MISS);
         hipLaunchKernelGGL(k_shade_miss, dim3(light_grid), dim3(BLOCK), 0, stream, s, p, tg, counters, base, bounce,
-                           light_sampling);
+                           light_sampling, hand_over);
         if (prof) prof->end(K_SHADE_MISS);
     }
     if (prof) prof->begin(K_SHADE_SURFACE);
@@ -1427,7 +1460,7 @@ hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const Sce
     if (shade_grid < 1) shade_grid = 1;
 #define CN_SHADE_LAUNCH(SB, LDS, SORT)                                                                      \
     hipLaunchKernelGGL((k_shade_surface<SB, LDS, SORT>), dim3(shade_grid), dim3(SB), 0, stream, s, p, tg, counters, \
-                       base, bounce, light_sampling)
+                       base, bounce, light_sampling, hand_over)
     switch (shape.shade_variant) {
         case SHADE_1024_LDS: CN_SHADE_LAUNCH(1024, true, false); break;
         case SHADE_512_LDS: CN_SHADE_LAUNCH(512, true, false); break;

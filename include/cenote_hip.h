@@ -365,10 +365,10 @@ typedef struct cn_launch_shape {
     uint32_t light_blocks;   /* most 256-lane workgroups of shade_miss, 1..65536 */
     uint32_t bvh_width;      /* 4 or 8: which of a scene's trees the traversal walks (a scene
                               * without an 8-wide tree is walked 4-wide) */
-    uint32_t tail_bounce;    /* 0: every bounce as wavefront stages; b in 1..255: after bounce b's
-                              * trace, one launch carries every live path through its remaining
-                              * bounces (the same films, bit for bit; waves with counters on keep
-                              * the stages) */
+    uint32_t tail_bounce;    /* 0: every bounce as wavefront stages; b in 1..255: after the trace of
+                              * bounce b, or of an earlier one with few rays, one launch carries
+                              * every live path through its remaining bounces (the same films, bit
+                              * for bit; waves with counters on keep the stages) */
 } cn_launch_shape;
 int cn_renderer_get_shape(cn_renderer* renderer, cn_launch_shape* out);
 int cn_renderer_set_shape(cn_renderer* renderer, const cn_launch_shape* shape);
