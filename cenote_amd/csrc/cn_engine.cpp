@@ -273,7 +273,7 @@ int enqueue_wave(cn_renderer* r, std::vector<HostJob> jobs, bool aov, const Wave
                 CN_HIP(launch_bounce(r->stream, r->shape, jobs[rg.g0].scene->view, pool, tg, counters, dev + rg.g0,
                                      uint32_t(rg.g1 - rg.g0), rg.base, rg.count, b, r->light_sampling, r->counting,
                                      range_tail, r->max_bounces, r->ctx->compute_units, r->profiler.get()));
-                if (b == range_tail) break;
+                if (b == tail_launch_bounce(range_tail, rg.count)) break;
             }
         }
         if (films) {

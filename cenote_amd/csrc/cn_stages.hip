@@ -80,6 +80,7 @@ __device__ __forceinline__ uint32_t queue_total(const uint32_t* counters, uint32
 // waves of a 720p session 9.3, 8.45, 8.45, 8.8; the veiled chart 2.87, 2.77,
 // 2.77, 2.79; waves of a million paths and more unchanged.
 constexpr uint32_t TAIL_PATHS = 16384;
+static_assert(TAIL_AT_ONCE <= TAIL_PATHS, "such a range's bounce 1 is handed over");
 __device__ __forceinline__ bool handed_over(const uint32_t* counters, uint32_t bounce, uint32_t hand_over) {
     return bounce > 0 && queue_total(counters, bounce, Q_RAY) <= hand_over;
 }
@@ -1390,7 +1391,7 @@ hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const Sce
                          const WaveTargets& tg, uint32_t* counters, const JobRecord* jobs, uint32_t job_count,
                          uint32_t base, uint32_t range_count, uint32_t bounce, uint32_t light_sampling, int counting,
                          uint32_t tail_bounce, uint32_t max_bounces, uint32_t compute_units, Profiler* prof) {
-    const bool tail = bounce == tail_bounce;
+    const bool tail = bounce == tail_launch_bounce(tail_bounce, range_count);
     const uint32_t hand_over = tail_bounce == UINT32_MAX ? 0u : TAIL_PATHS;
     const uint32_t light_grid = grid_for(range_count, shape.light_blocks);
     // Bounce b's rays and bounce b-1's shadow rays share one launch; the
@@ -1440,10 +1441,10 @@ hipError_t launch_bounce(hipStream_t stream, const LaunchShape& shape, const Sce
         if (prof) prof->begin(K_TAIL);
         if (wide)
             hipLaunchKernelGGL(k_tail<true>, dim3(tail_grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg, counters,
-                               counters + tail_claim_index(max_bounces), base, bounce, light_sampling, hand_over);
+                               counters + tail_claim_index(max_bounces), base, tail_bounce, light_sampling, hand_over);
         else
             hipLaunchKernelGGL(k_tail<false>, dim3(tail_grid), dim3(TRAVERSAL_BLOCK), 0, stream, s, p, tg, counters,
-                               counters + tail_claim_index(max_bounces), base, bounce, light_sampling, hand_over);
+                               counters + tail_claim_index(max_bounces), base, tail_bounce, light_sampling, hand_over);
         if (prof) prof->end(K_TAIL);
         return hipGetLastError();
     }
