@@ -57,7 +57,6 @@ __host__ __device__ __forceinline__ bool any_positive(v3 v) { return v.x > 0.0f 
 __host__ __device__ __forceinline__ v3 vfma(v3 a, v3 b, v3 c) {
     return {fmaf(a.x, b.x, c.x), fmaf(a.y, b.y, c.y), fmaf(a.z, b.z, c.z)};
 }
-__host__ __device__ __forceinline__ float mean3(v3 v) { return (v.x + v.y + v.z) / 3.0f; }
 __host__ __device__ __forceinline__ float signf(float x) { return x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f); }
 __host__ __device__ __forceinline__ v3 xyz(float4 v) { return {v.x, v.y, v.z}; }
 __host__ __device__ __forceinline__ float4 F4(v3 v, float w) { return make_float4(v.x, v.y, v.z, w); }

@@ -81,6 +81,13 @@ void land(const Piece& p, const float* in) {
 
 static int read_pieces(int device, Readback& rb, const ReadArray* arrays, int n) {
     constexpr size_t SLOT_VALUES = Readback::SLOT / sizeof(float);
+    // An array by way of one pageable copy.
+    auto whole = [](const ReadArray& a) {
+        std::vector<float> values(a.count);
+        CN_HIP(hipMemcpy(values.data(), a.src, a.count * sizeof(float), hipMemcpyDeviceToHost));
+        land({&a, 0, a.count}, values.data());
+        return int(CN_OK);
+    };
     std::vector<Piece> pieces;
     for (int i = 0; i < n; ++i) {
         const ReadArray& a = arrays[i];
@@ -89,10 +96,8 @@ static int read_pieces(int device, Readback& rb, const ReadArray* arrays, int n)
         if (a.width) {
             const size_t band = size_t(a.width) * 8 * a.lanes;
             if (band > SLOT_VALUES) {
-                // A band that fills more than a slot: by way of a whole copy.
-                std::vector<float> whole(a.count);
-                CN_HIP(hipMemcpy(whole.data(), a.src, a.count * sizeof(float), hipMemcpyDeviceToHost));
-                land({&a, 0, a.count}, whole.data());
+                // A band that fills more than a slot.
+                if (int e = whole(a)) return e;
                 continue;
             }
             step = SLOT_VALUES / band * band;
@@ -102,15 +107,27 @@ static int read_pieces(int device, Readback& rb, const ReadArray* arrays, int n)
     }
     if (pieces.empty()) return CN_OK;
     std::lock_guard<std::mutex> lock(rb.busy);
-    CN_HIP(rb.prepare());
+    if (rb.prepare() != hipSuccess) {
+        // No pinned memory (or streams) to be had.
+        (void)hipGetLastError();
+        const ReadArray* last = nullptr;
+        for (const Piece& p : pieces) {
+            if (p.a == last) continue;
+            last = p.a;
+            if (int e = whole(*last)) return e;
+        }
+        return CN_OK;
+    }
     auto copy = [&](int worker, int slot, const Piece& p) {
         return hipMemcpyAsync(rb.slots + Readback::SLOT * slot, p.a->src + p.first, p.count * sizeof(float),
                               hipMemcpyDeviceToHost, rb.streams[worker]);
     };
     auto staged = [&](int slot) { return reinterpret_cast<const float*>(rb.slots + Readback::SLOT * slot); };
     if (pieces.size() <= 4) {
-        for (size_t k = 0; k < pieces.size(); ++k) CN_HIP(copy(0, int(k), pieces[k]));
-        CN_HIP(hipStreamSynchronize(rb.streams[0]));
+        hipError_t e = hipSuccess;
+        for (size_t k = 0; k < pieces.size() && e == hipSuccess; ++k) e = copy(0, int(k), pieces[k]);
+        const hipError_t done = hipStreamSynchronize(rb.streams[0]);  // also before the slots are let go
+        CN_HIP(e != hipSuccess ? e : done);
         for (size_t k = 0; k < pieces.size(); ++k) land(pieces[k], staged(int(k)));
         return CN_OK;
     }

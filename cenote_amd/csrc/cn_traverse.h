@@ -4,7 +4,10 @@
 // units).
 //
 // One lane per ray, closest-first descent with a short stack (LDS, spilling
-// to HBM), and the speculative while-while schedule of Aila & Laine
+// to HBM). Queues of rays are walked by walk_many: a wave refills finished
+// lanes and votes on every step's kind. Rays that a lane brings by itself
+// (the tail's, first hits, counting camera rays, attenuation) are walked by
+// walk, on the speculative while-while schedule of Aila & Laine
 // ("Understanding the Efficiency of Ray Traversal on GPUs", HPG 2009): a
 // lane that reaches a leaf postpones it and keeps descending until every
 // lane of the wave64 holds a leaf, so leaf tests run with full SIMD lanes.
@@ -699,37 +702,15 @@ __device__ __forceinline__ bool visibility_leaf(const SceneView& s, const Ray& w
     return false;
 }
 
-template <bool W8>
-__device__ inline float shadow_attenuation(const SceneView& s, const Ray& r, float t_end,
-                                           uint32_t target_inst, uint32_t target_prim, Stack& st,
-                                           uint32_t& nodes_visited);
-
 // A next-event connection's visibility (trace_shadow.slang:41-71): visible
 // iff nothing solid commits within tmax or the committed hit is the target
-// (instance, primitive). Returns the attenuation (0 when occluded or
-// attenuated below 1e-4): the transmittance of every fractional-opacity
-// crossing in front of the connection's end, taken in an order-free form
-// (exp2_fixed of a sum of fixed-point logarithms). A solid non-target hit
-// nearer than `t_early` occludes without looking further.
-template <bool W8>
-__device__ __forceinline__ float trace_visibility(const SceneView& s, v3 o, v3 d, float tmax, uint32_t target_inst,
-                                                  uint32_t target_prim, float t_early, Stack& st,
-                                                  uint32_t& nodes_visited, uint32_t& tris_tested) {
-    const Ray r = make_ray(o, d);
-    TraceHit best = no_hit(tmax);
-    bool occluded = false, translucent = false;
-    walk(tree_of<W8>(s), r, best.t, st, nodes_visited, [&](uint32_t ref) {
-        occluded = visibility_leaf(s, r, ref, target_inst, target_prim, t_early, best, translucent, tris_tested);
-        return occluded;
-    });
-    if (occluded) return 0.0f;
-    if (best.hit() && !(best.inst == target_inst && best.prim == target_prim)) return 0.0f;
-    if (!translucent) return 1.0f;
-    return shadow_attenuation<W8>(s, r, best.t, target_inst, target_prim, st, nodes_visited);
-}
-
-// The rare path of a visible connection that crossed fractional-opacity
-// geometry: one more walk over [0, t_end) adds each non-target crossing's
+// (instance, primitive). What remains is its attenuation (0 below 1e-4): the
+// transmittance of every fractional-opacity crossing in front of the
+// connection's end, taken in an order-free form (exp2_fixed of a sum of
+// fixed-point logarithms).
+//
+// This is the rare path of a visible connection that crossed fractional-
+// opacity geometry: one more walk over [0, t_end) adds each non-target crossing's
 // fixed-point log2 transmittance (the instance record's `log2_transmittance`,
 // rounded on the host) and stops once the sum is below the cutoff. Integer
 // adds make the result independent of the walk's order.
@@ -772,7 +753,8 @@ __device__ inline float shadow_attenuation(const SceneView& s, const Ray& r, flo
 // on the 2M-triangle scene seen from inside). Weighting the vote 2:1 for nodes
 // took 40% longer, 2:1 for leaves 1%; keeping 32, 40, 48 or 54 lanes walking
 // measured 26.3, 26.3, 26.4 and 26.8 ms there and 8.2, 8.3, 8.7 and 9.0 on
-// the chart, whose rays are short.
+// the chart, whose rays are short (these with leaves of up to 8 triangles;
+// with 4, 24.2 and 7.6 ms).
 //
 // take(i) starts entry i in the calling lane: sets the lane's ray and bound;
 // test(triangle) tests one triangle (it may shrink the bound) and returns true
