@@ -583,7 +583,7 @@ def _base_name(kernel_name):
 def _stage_of(kernel_name):
     """The stage a dispatched kernel belongs to, or None. Counting-pass
     traversal kernels (COUNT = true) belong to no stage."""
-    base = _base_name(kernel_name)
+    base = _base_name(kernel_name).replace("k_trace_camera", "k_trace")  # bounce 0's trace launch
     for stage, sym in KERNEL_SYMBOLS.items():
         if sym + "<" in base or base.endswith(sym):
             if stage == "trace" and (sym + "<true") in base:
@@ -619,7 +619,7 @@ def reduce_profile(directory, name, steps, capacity, tail=0):
         stage = _stage_of(d["kernel"])
         if stage is not None:
             stages[stage].append(d)
-        elif "k_trace<true" not in d["kernel"]:
+        elif "k_trace<true" not in d["kernel"] and "k_trace_camera<true" not in d["kernel"]:
             others.setdefault(_short(d["kernel"]), []).append(d)
 
     def averages(ds):
