@@ -355,8 +355,9 @@ __global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu
 // lanes active when every lane kept its ray until its wave was done). Refilled
 // and voted, that launch (29M rays and 6M connections) went from 14.1 to 9.3
 // ms; the frame's trace time from 32.8 to 26.2 ms there, 13.6 to 11.7 on the
-// outside view, 10.7 to 8.1 on the chart. Eight waves per SIMD (64 VGPRs; LDS
-// 8 x 18 KB per CU) measured 25.8 ms against 26.0 at seven and at six.
+// outside view, 10.7 to 8.1 on the chart (8.6; 23.4, 10.7 and 7.5 over the
+// present, finer tree). Eight waves per SIMD (64 VGPRs; LDS 8 x 18 KB per CU)
+// measured 25.8 ms against 26.0 at seven and at six.
 // Chunks: 256 to 1,024 entries within 2% (512 kept); a fixed share per wave
 // instead of claims 27.8 ms. The grid of 16,384 blocks that this replaces took
 // 80 us to dispatch even for a few hundred rays; a launch of 800 rays now
@@ -934,7 +935,7 @@ __global__ __launch_bounds__(SB) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // connection, so the two walks of a bounce overlap instead of following
 // one another (a deep path's latency is a chain of dependent fetches; on
 // the 2M-triangle scene the tail took 1.54 ms per frame this way against
-// 2.21 ms with one lane per path). The owner adds the connection's light
+// 2.21 ms with one lane per path, before it was spread as told below). The owner adds the connection's light
 // after both walks and before it shades the next hit.
 template <bool W8>
 __global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu(TAIL_WAVES))) void k_tail(
