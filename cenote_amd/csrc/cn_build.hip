@@ -39,7 +39,8 @@ constexpr uint32_t CHUNK = 8192;       // triangles per workgroup in the device-
 constexpr uint32_t SMALL_TASK = 2048;  // ranges at most this large are built by one workgroup
 constexpr uint32_t SMALL_STACK = 32;   // ample: smaller-first keeps it under log2(SMALL_TASK) + 1
 constexpr uint32_t WAVE_TASK = 64;     // ranges at most this large are built by one wave, a triangle a lane
-static_assert(WAVE_TASK >= BVH_LEAF_SIZE && WAVE_TASK < SMALL_TASK, "only a wave makes leaves");
+static_assert(WAVE_TASK >= BVH_RULES.leaf_size && WAVE_TASK >= BVH_COARSE_RULES.leaf_size && WAVE_TASK < SMALL_TASK,
+              "only a wave makes leaves");
 
 // Floats as order-preserving unsigned integers, so integer atomic min/max
 // fold float bounds exactly.
@@ -237,20 +238,21 @@ __device__ void k_chunk_scatter_body(const Chunk& ch, const TaskSplit* __restric
 // the sequential sweep computes, since a fold of boxes is the same in any
 // order — and a (cost, candidate index) minimum picks the candidate the
 // sequential sweep keeps (the first of the lowest cost). Thread 0 returns
-// the decision (with the left count) in `*out`. Every thread of the block
-// must call it.
+// the split (with the left count) in `*out`: ranges this large, more than
+// WAVE_TASK triangles, never make a leaf. Every thread of the block must call
+// it.
 struct Decision {
     SplitDecision d;
     uint32_t left;  // primitives in bins 0..split of the chosen axis
 };
 
-__device__ void decide_block(const Box3 (*fbins)[BVH_BINS], const uint32_t (*fcounts)[BVH_BINS], const Box3& box,
-                             const Box3& cbox, uint32_t n, float* red_cost, uint32_t* red_idx, uint32_t* red_left,
+__device__ void decide_block(const Box3 (*fbins)[BVH_BINS], const uint32_t (*fcounts)[BVH_BINS], const Box3& cbox,
+                             float* red_cost, uint32_t* red_idx, uint32_t* red_left,
                              Decision* out) {
     const uint32_t tid = threadIdx.x;
     float cost = INFINITY;
     uint32_t idx = 0xffffffffu, lcnt = 0;
-    if (tid < 3 * BVH_BINS && n > 1) {
+    if (tid < 3 * BVH_BINS) {
         const int axis = int(tid / BVH_BINS), b = int(tid % BVH_BINS);
         if (b < BVH_BINS - 1 && cbox.hi[axis] - cbox.lo[axis] > 0.0f) {
             Box3 lacc = Box3::empty(), racc = Box3::empty();
@@ -299,18 +301,10 @@ __device__ void decide_block(const Box3 (*fbins)[BVH_BINS], const uint32_t (*fco
         Decision r;
         r.d = SplitDecision{0, -1, 0};
         r.left = 0;
-        if (n <= 1) {
-            r.d.leaf = 1;
-        } else {
-            if (bi != 0xffffffffu) {
-                r.d.axis = int(bi / BVH_BINS);
-                r.d.split = int(bi % BVH_BINS);
-                r.left = bl;
-            }
-            const float parent_area = box.area();
-            const float leaf_cost = float(n);
-            const float split_cost = BVH_NODE_COST + (parent_area > 0.0f ? best / parent_area : 0.0f);
-            if (n <= BVH_LEAF_SIZE && (r.d.axis < 0 || leaf_cost <= split_cost)) r.d.leaf = 1;
+        if (bi != 0xffffffffu) {
+            r.d.axis = int(bi / BVH_BINS);
+            r.d.split = int(bi % BVH_BINS);
+            r.left = bl;
         }
         *out = r;
     }
@@ -501,7 +495,7 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_level_decide(const Task* __rest
         }
     }
     __syncthreads();
-    decide_block(fbins, fcounts, box, cbox, m, red_cost, red_idx, red_left, &dec);
+    decide_block(fbins, fcounts, cbox, red_cost, red_idx, red_left, &dec);
     if (threadIdx.x != 0) return;
     TaskSplit sp{task.begin, m, 1u, 0u, 0, m / 2, 0.0f, 0.0f};
     if (dec.d.axis >= 0 && dec.left > 0 && dec.left < m) {
@@ -513,7 +507,7 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_level_decide(const Task* __rest
         sp.scale = bvh_scale(cbox.lo[dec.d.axis], cbox.hi[dec.d.axis]);
     }
     splits[k] = sp;
-    // Ranges this large always split (a leaf holds at most BVH_LEAF_SIZE triangles).
+    // Ranges this large always split (decide_block).
     const uint32_t ids = atomicAdd(&state[S_NODES], 2u);
     BinaryNode node;
     node.box = box;
@@ -735,9 +729,9 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_small_build(const Task* __restr
             cbox.lo[k] = o2f(red[6 + k]);
             cbox.hi[k] = o2f(red[9 + k]);
         }
-        decide_block(fbins, fcounts, box, cbox, m, red_cost, red_idx, red_left, &dec);
+        decide_block(fbins, fcounts, cbox, red_cost, red_idx, red_left, &dec);
         if (threadIdx.x == 0) {
-            // Ranges this large always split (a leaf holds at most BVH_LEAF_SIZE triangles).
+            // Ranges this large always split (decide_block).
             uint32_t l = m / 2;
             int bin_mode = 0;
             if (dec.d.axis >= 0 && dec.left > 0 && dec.left < m) {
@@ -809,7 +803,8 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_small_build(const Task* __restr
 // at most WAVE_TASK levels follow. Bound by the loops' shuffles: 1.7 ms for a
 // million triangles, after 0.7 ms of k_small_build.
 __global__ __launch_bounds__(BUILD_BLOCK) void k_wave_build(const uint32_t* __restrict__ list, PrimArrays p,
-                                                            uint32_t* order, BinaryNode* nodes, uint32_t* state) {
+                                                            uint32_t* order, BinaryNode* nodes, uint32_t* state,
+                                                            BvhRules rules) {
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t below = (uint64_t(1) << lane) - 1;
     const uint32_t tasks = state[S_WAVE];
@@ -901,9 +896,9 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_wave_build(const uint32_t* __re
 
             // bvh_decide's choice, and the children or the leaf.
             const float parent_area = box.area();
-            const float split_cost = BVH_NODE_COST + (parent_area > 0.0f ? best / parent_area : 0.0f);
+            const float split_cost = rules.node_cost + (parent_area > 0.0f ? best / parent_area : 0.0f);
             const bool binned = at != 0xffffffffu;
-            const bool leaf = m <= 1 || (m <= BVH_LEAF_SIZE && (!binned || float(m) <= split_cost));
+            const bool leaf = m <= 1 || (m <= rules.leaf_size && (!binned || float(m) <= split_cost));
             const bool splits = m > 0 && !leaf;
             const uint64_t leaders = __ballot(splits && lane == first);
             uint32_t base = 0;
@@ -1381,97 +1376,110 @@ bool build_bvh_device(const DeviceTriangles& input, uint32_t max_stack, Bvh4* ou
     BUILD_CHECK(hipMemcpy(d_first, first.data(), 4 * first.size(), hipMemcpyHostToDevice));
     hipLaunchKernelGGL(k_world_triangles, dim3(blocks_for(n)), dim3(BUILD_BLOCK), 0, nullptr, input.mesh_tris,
                        input.instances, d_flags, d_first, instances, n, d_in);
-    {
-        uint32_t init[S_WORDS] = {};
-        init[S_NODES] = 1;
-        const Task root{0, n, 0, 0};
-        if (n > SMALL_TASK) {
-            init[S_BIG] = 1;
-            BUILD_CHECK(hipMemcpy(big[0], &root, sizeof(root), hipMemcpyHostToDevice));
-        } else {
-            init[S_SMALL] = 1;
-            BUILD_CHECK(hipMemcpy(small, &root, sizeof(root), hipMemcpyHostToDevice));
+    // The binary tree by `rules`.
+    const auto grow = [&](const BvhRules& rules) {
+        {
+            uint32_t init[S_WORDS] = {};
+            init[S_NODES] = 1;
+            const Task root{0, n, 0, 0};
+            if (n > SMALL_TASK) {
+                init[S_BIG] = 1;
+                BUILD_CHECK(hipMemcpy(big[0], &root, sizeof(root), hipMemcpyHostToDevice));
+            } else {
+                init[S_SMALL] = 1;
+                BUILD_CHECK(hipMemcpy(small, &root, sizeof(root), hipMemcpyHostToDevice));
+            }
+            BUILD_CHECK(hipMemcpy(state, init, sizeof(init), hipMemcpyHostToDevice));
         }
-        BUILD_CHECK(hipMemcpy(state, init, sizeof(init), hipMemcpyHostToDevice));
-    }
-    hipLaunchKernelGGL(k_prims, dim3(blocks_for(n)), dim3(BUILD_BLOCK), 0, nullptr, d_in, n, p, order,
-                       state + S_MAX_ABS, state + S_BAD);
-    BUILD_CHECK(hipGetLastError());
+        hipLaunchKernelGGL(k_prims, dim3(blocks_for(n)), dim3(BUILD_BLOCK), 0, nullptr, d_in, n, p, order,
+                           state + S_MAX_ABS, state + S_BAD);
+        BUILD_CHECK(hipGetLastError());
 
-    // Top levels, eight at a time between reads of the device's task count:
-    // every decision is made on the device from device-resident bins.
-    uint32_t st[S_WORDS];
-    const uint32_t init_grid = std::min<uint32_t>(blocks_for(size_t(big_cap) * TBIN), 4096);
-    int cur = 0;
-    for (uint32_t batch = 0;; ++batch) {
+        // Top levels, eight at a time between reads of the device's task count:
+        // every decision is made on the device from device-resident bins.
+        uint32_t st[S_WORDS];
+        const uint32_t init_grid = std::min<uint32_t>(blocks_for(size_t(big_cap) * TBIN), 4096);
+        int cur = 0;
+        for (uint32_t batch = 0;; ++batch) {
+            BUILD_CHECK(hipMemcpy(st, state, sizeof(st), hipMemcpyDeviceToHost));
+            if (st[S_BAD]) {
+                *error = "scene geometry holds a non-finite vertex";
+                return false;
+            }
+            if (st[S_OVERFLOW]) {
+                *error = "device BVH build: task list overflow (" + std::to_string(st[S_OVERFLOW]) + ")";
+                return false;
+            }
+            if (st[S_BIG] == 0) break;
+            if (batch > n) {
+                *error = "device BVH build: the top levels did not finish";
+                return false;
+            }
+            for (int level = 0; level < 8; ++level) {
+                hipLaunchKernelGGL(k_level_chunks, dim3(1), dim3(BUILD_BLOCK), 0, nullptr, big[cur], state, chunks,
+                                   chunk_first, chunk_cap);
+                hipLaunchKernelGGL(k_level_init, dim3(init_grid), dim3(BUILD_BLOCK), 0, nullptr, state, tb, bins);
+                hipLaunchKernelGGL(k_level_bounds, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state, p,
+                                   order, tb);
+                hipLaunchKernelGGL(k_level_bins, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state, p,
+                                   order, tb, bins);
+                hipLaunchKernelGGL(k_level_decide, dim3(big_cap), dim3(BUILD_BLOCK), 0, nullptr, big[cur], state, tb,
+                                   bins, splits, d_nodes, big[1 - cur], small, big_cap, small_cap);
+                hipLaunchKernelGGL(k_level_count, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state,
+                                   splits, p, order, lefts);
+                hipLaunchKernelGGL(k_level_bases, dim3(blocks_for(big_cap)), dim3(BUILD_BLOCK), 0, nullptr,
+                                   chunk_first, state, chunks, splits, lefts, lbase, rbase);
+                hipLaunchKernelGGL(k_level_scatter, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state,
+                                   splits, p, order, lbase, rbase, order_tmp);
+                hipLaunchKernelGGL(k_level_copy, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state,
+                                   order_tmp, order);
+                hipLaunchKernelGGL(k_level_advance, dim3(1), dim3(1), 0, nullptr, state);
+                cur = 1 - cur;
+            }
+            BUILD_CHECK(hipGetLastError());
+        }
+
+        // Subtrees, one workgroup each, then one wave each; the waves' list lies
+        // in the scatter's second order, which nothing reads any more (its ranges
+        // are disjoint, so it has at most n entries).
+        if (st[S_SMALL] > 0) {
+            hipLaunchKernelGGL(k_small_build, dim3(st[S_SMALL]), dim3(BUILD_BLOCK), 0, nullptr, small, state + S_SMALL,
+                               p, order, d_nodes, order_tmp, n, state);
+            hipLaunchKernelGGL(k_wave_build, dim3(std::min<uint32_t>(blocks_for(n), 2048)), dim3(BUILD_BLOCK), 0,
+                               nullptr, order_tmp, p, order, d_nodes, state, rules);
+            BUILD_CHECK(hipGetLastError());
+        }
         BUILD_CHECK(hipMemcpy(st, state, sizeof(st), hipMemcpyDeviceToHost));
-        if (st[S_BAD]) {
-            *error = "scene geometry holds a non-finite vertex";
-            return false;
-        }
         if (st[S_OVERFLOW]) {
-            *error = "device BVH build: task list overflow (" + std::to_string(st[S_OVERFLOW]) + ")";
+            *error = "device BVH build: subtree stack overflow";
             return false;
         }
-        if (st[S_BIG] == 0) break;
-        if (batch > n) {
-            *error = "device BVH build: the top levels did not finish";
+        if (st[S_NODES] > 2 * size_t(n)) {
+            *error = "device BVH build: node count out of range";
             return false;
         }
-        for (int level = 0; level < 8; ++level) {
-            hipLaunchKernelGGL(k_level_chunks, dim3(1), dim3(BUILD_BLOCK), 0, nullptr, big[cur], state, chunks,
-                               chunk_first, chunk_cap);
-            hipLaunchKernelGGL(k_level_init, dim3(init_grid), dim3(BUILD_BLOCK), 0, nullptr, state, tb, bins);
-            hipLaunchKernelGGL(k_level_bounds, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state, p,
-                               order, tb);
-            hipLaunchKernelGGL(k_level_bins, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state, p, order,
-                               tb, bins);
-            hipLaunchKernelGGL(k_level_decide, dim3(big_cap), dim3(BUILD_BLOCK), 0, nullptr, big[cur], state, tb,
-                               bins, splits, d_nodes, big[1 - cur], small, big_cap, small_cap);
-            hipLaunchKernelGGL(k_level_count, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state, splits,
-                               p, order, lefts);
-            hipLaunchKernelGGL(k_level_bases, dim3(blocks_for(big_cap)), dim3(BUILD_BLOCK), 0, nullptr, chunk_first,
-                               state, chunks, splits, lefts, lbase, rbase);
-            hipLaunchKernelGGL(k_level_scatter, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state, splits,
-                               p, order, lbase, rbase, order_tmp);
-            hipLaunchKernelGGL(k_level_copy, dim3(chunk_cap), dim3(BUILD_BLOCK), 0, nullptr, chunks, state,
-                               order_tmp, order);
-            hipLaunchKernelGGL(k_level_advance, dim3(1), dim3(1), 0, nullptr, state);
-            cur = 1 - cur;
-        }
-        BUILD_CHECK(hipGetLastError());
-    }
-
-    // Subtrees, one workgroup each, then one wave each; the waves' list lies
-    // in the scatter's second order, which nothing reads any more (its ranges
-    // are disjoint, so it has at most n entries).
-    if (st[S_SMALL] > 0) {
-        hipLaunchKernelGGL(k_small_build, dim3(st[S_SMALL]), dim3(BUILD_BLOCK), 0, nullptr, small, state + S_SMALL, p,
-                           order, d_nodes, order_tmp, n, state);
-        hipLaunchKernelGGL(k_wave_build, dim3(std::min<uint32_t>(blocks_for(n), 2048)), dim3(BUILD_BLOCK), 0, nullptr,
-                           order_tmp, p, order, d_nodes, state);
-        BUILD_CHECK(hipGetLastError());
-    }
-    BUILD_CHECK(hipMemcpy(st, state, sizeof(st), hipMemcpyDeviceToHost));
-    if (st[S_OVERFLOW]) {
-        *error = "device BVH build: subtree stack overflow";
-        return false;
-    }
-    if (st[S_NODES] > 2 * size_t(n)) {
-        *error = "device BVH build: node count out of range";
-        return false;
-    }
-    float max_abs;
-    std::memcpy(&max_abs, &st[S_MAX_ABS], 4);
-    (void)max_abs;
+        return true;
+    };
+    if (!grow(BVH_RULES)) return false;
 
     // Collapse to 4-wide nodes (preorder numbering, as the host collapse),
-    // full precision and quantized, then to 8-wide quantized nodes.
+    // full precision and quantized, then to 8-wide quantized nodes. A tree too
+    // deep is grown once more, as by the host builder.
     WideTmp<4>* wide4 = nullptr;
     uint32_t* idx4 = nullptr;
     uint32_t depth4 = 0, count4 = 0;
     bool deep = false;
-    if (!collapse_device<4>(d_nodes, n, state, max_stack / 3, s, &wide4, &idx4, &depth4, &count4, &deep, error)) {
+    const auto collapse = [&] {
+        deep = false;
+        return collapse_device<4>(d_nodes, n, state, max_stack / 3, s, &wide4, &idx4, &depth4, &count4, &deep,
+                                  error);
+    };
+    bool whole = collapse();
+    if (!whole && deep) {
+        if (!grow(BVH_COARSE_RULES)) return false;
+        whole = collapse();
+    }
+    if (!whole) {
         if (deep) *error = "BVH too deep for the traversal stack (depth " + std::to_string(depth4) + ")";
         return false;
     }

@@ -34,10 +34,11 @@ struct Builder {
     const std::vector<Prim>& prims;
     std::vector<uint32_t>& order;
     std::vector<BNode>& nodes;
+    const BvhRules& rules;
     std::atomic<uint32_t> next{1};
 
-    Builder(const std::vector<Prim>& p, std::vector<uint32_t>& o, std::vector<BNode>& n)
-        : prims(p), order(o), nodes(n) {}
+    Builder(const std::vector<Prim>& p, std::vector<uint32_t>& o, std::vector<BNode>& n, const BvhRules& r)
+        : prims(p), order(o), nodes(n), rules(r) {}
 
     uint32_t alloc2() { return next.fetch_add(2); }
 
@@ -67,7 +68,7 @@ struct Builder {
                 ++counts[axis][b];
             }
         }
-        const SplitDecision d = bvh_decide(box, cbox, bins, counts, n);
+        const SplitDecision d = bvh_decide(box, cbox, bins, counts, n, rules);
         if (d.leaf) {
             out.first = begin;
             out.count = n;
@@ -334,12 +335,16 @@ bool build_bvh4(const std::vector<WorldTriangle>& input, uint32_t max_stack, Bvh
         return false;
     }
     std::vector<uint32_t> order(n);
-    for (uint32_t i = 0; i < n; ++i) order[i] = i;
-    std::vector<BNode> bnodes(2 * size_t(n));
-    Builder builder(prims, order, bnodes);
-    builder.build(0, 0, n, 0);
-    bnodes.resize(builder.next.load());
-    if (!collapse_to_bvh4(bnodes, max_abs, max_stack, out, error)) return false;
+    std::vector<BNode> bnodes;
+    const auto grow = [&](const BvhRules& rules) {
+        for (uint32_t i = 0; i < n; ++i) order[i] = i;
+        bnodes.assign(2 * size_t(n), BNode{});
+        Builder builder(prims, order, bnodes, rules);
+        builder.build(0, 0, n, 0);
+        bnodes.resize(builder.next.load());
+        return collapse_to_bvh4(bnodes, max_abs, max_stack, out, error);
+    };
+    if (!grow(BVH_RULES) && !grow(BVH_COARSE_RULES)) return false;
     collapse_to_bvh8(bnodes, max_abs, max_stack, out);
 
     out->tris.resize(n);

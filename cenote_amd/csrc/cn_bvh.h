@@ -38,10 +38,10 @@ struct BinaryNode {
 };
 static_assert(sizeof(BinaryNode) == 40, "device and host share this layout");
 
-// Binned-SAH binary build (32 bins on the three axes, leaves of <= 4
-// triangles), collapsed to 4-wide nodes by repeatedly opening the child of
-// largest surface area. Returns false with a message when the tree would
-// be deeper than the traversal stack allows.
+// Binned-SAH binary build (32 bins on the three axes, leaves by BVH_RULES),
+// collapsed to 4-wide nodes by repeatedly opening the child of largest surface
+// area. A tree deeper than the traversal stack allows is grown again by
+// BVH_COARSE_RULES; returns false with a message when that is too deep too.
 bool build_bvh4(const std::vector<WorldTriangle>& input, uint32_t max_stack, Bvh4* out, std::string* error);
 
 // The collapse step alone, from a binary tree rooted at node 0 (nodes may

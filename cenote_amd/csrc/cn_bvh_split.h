@@ -14,7 +14,14 @@
 namespace cn {
 
 constexpr int BVH_BINS = 32;
-// The SAH's traversal term and the largest leaf, for the voted walk of the
+
+// What a tree is grown by: the largest leaf, and the SAH's traversal term (a
+// triangle test costs 1).
+struct BvhRules {
+    uint32_t leaf_size;
+    float node_cost;
+};
+// The rules of nearly every tree, for the voted walk of the
 // trace kernel: a triangle step of a wave costs about as much as a node step
 // (90 to 150 instructions against 140, and both end the vote's turn), and its
 // lanes wait on it, so small leaves pay. Trace ms per frame at node cost 2,
@@ -23,8 +30,10 @@ constexpr int BVH_BINS = 32;
 // triangles make a few leaves, 0.605 and then 0.465. Leaves of 8, 4, 3 and 2
 // measured within 2% of one another below cost 1; 4 keeps the tree smaller
 // than 2.
-constexpr uint32_t BVH_LEAF_SIZE = 4;
-constexpr float BVH_NODE_COST = 0.7f;
+constexpr BvhRules BVH_RULES{4, 0.7f};
+// Larger leaves make a tree of fewer nodes that ends a level or two earlier:
+// for a scene whose tree by the rules above does not fit the traversal.
+constexpr BvhRules BVH_COARSE_RULES{8, 2.0f};
 
 struct Box3 {
     float lo[3], hi[3];
@@ -64,13 +73,13 @@ struct SplitDecision {
     int split;  // bins 0..split go left
 };
 
-// Binned SAH over the three axes (32 bins; leaves of <= 4 triangles when a
-// leaf is no costlier than the best split, a triangle test costing 1 and a
-// node step BVH_NODE_COST). `bins`/`counts` hold the
+// Binned SAH over the three axes (32 bins; a leaf where the rules allow one of
+// `n` triangles and none of the splits is cheaper). `bins`/`counts` hold the
 // range's per-axis bins; axes whose centroid extent is not positive are
 // skipped (their bins are ignored).
 __host__ __device__ inline SplitDecision bvh_decide(const Box3& box, const Box3& cbox, const Box3 (*bins)[BVH_BINS],
-                                                    const uint32_t (*counts)[BVH_BINS], uint32_t n) {
+                                                    const uint32_t (*counts)[BVH_BINS], uint32_t n,
+                                                    const BvhRules& rules) {
     SplitDecision d{0, -1, 0};
     if (n <= 1) {
         d.leaf = 1;
@@ -106,8 +115,8 @@ __host__ __device__ inline SplitDecision bvh_decide(const Box3& box, const Box3&
     }
     const float parent_area = box.area();
     const float leaf_cost = float(n);
-    const float split_cost = BVH_NODE_COST + (parent_area > 0.0f ? best_cost / parent_area : 0.0f);
-    if (n <= BVH_LEAF_SIZE && (d.axis < 0 || leaf_cost <= split_cost)) d.leaf = 1;
+    const float split_cost = rules.node_cost + (parent_area > 0.0f ? best_cost / parent_area : 0.0f);
+    if (n <= rules.leaf_size && (d.axis < 0 || leaf_cost <= split_cost)) d.leaf = 1;
     return d;
 }
 
