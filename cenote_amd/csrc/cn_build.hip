@@ -1309,7 +1309,7 @@ bool collapse_device(const BinaryNode* d_nodes, uint32_t n, uint32_t* state, uin
 
 }  // namespace
 
-bool build_bvh_device(const DeviceTriangles& input, uint32_t max_stack, Bvh4* out, DeviceBvh* dev,
+bool build_bvh_device(const DeviceTriangles& input, const BvhLimits& limits, Bvh4* out, DeviceBvh* dev,
                       std::string* error) {
     const auto t0 = std::chrono::steady_clock::now();
     *dev = DeviceBvh{};
@@ -1463,24 +1463,28 @@ bool build_bvh_device(const DeviceTriangles& input, uint32_t max_stack, Bvh4* ou
     if (!grow(BVH_RULES)) return false;
 
     // Collapse to 4-wide nodes (preorder numbering, as the host collapse),
-    // full precision and quantized, then to 8-wide quantized nodes. A tree too
-    // deep is grown once more, as by the host builder.
+    // full precision and quantized, then to 8-wide quantized nodes. A tree past
+    // the limits is grown once more, as by the host builder.
     WideTmp<4>* wide4 = nullptr;
     uint32_t* idx4 = nullptr;
     uint32_t depth4 = 0, count4 = 0;
     bool deep = false;
     const auto collapse = [&] {
         deep = false;
-        return collapse_device<4>(d_nodes, n, state, max_stack / 3, s, &wide4, &idx4, &depth4, &count4, &deep,
+        return collapse_device<4>(d_nodes, n, state, limits.max_stack / 3, s, &wide4, &idx4, &depth4, &count4, &deep,
                                   error);
     };
     bool whole = collapse();
-    if (!whole && deep) {
+    if (whole ? count4 > limits.nodes4 : deep) {
         if (!grow(BVH_COARSE_RULES)) return false;
         whole = collapse();
     }
     if (!whole) {
         if (deep) *error = "BVH too deep for the traversal stack (depth " + std::to_string(depth4) + ")";
+        return false;
+    }
+    if (count4 > limits.nodes4) {
+        *error = "BVH of more nodes than the traversal addresses (" + std::to_string(count4) + ")";
         return false;
     }
     BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&dev->full), sizeof(BvhNode4) * count4));
@@ -1496,14 +1500,17 @@ bool build_bvh_device(const DeviceTriangles& input, uint32_t max_stack, Bvh4* ou
     uint32_t* idx8 = nullptr;
     uint32_t depth8 = 0, count8 = 0;
     out->max_depth8 = 0;
-    if (collapse_device<8>(d_nodes, n, state, max_stack / 7, s, &wide8, &idx8, &depth8, &count8, &deep, error)) {
-        BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&dev->nodes8), sizeof(BvhNode8Q) * count8));
-        dev->node8_count = count8;
-        const uint32_t grid8 = std::min<uint32_t>(blocks_for(count8), 2048);
-        hipLaunchKernelGGL(k_collapse_write8, dim3(grid8), dim3(BUILD_BLOCK), 0, nullptr, d_nodes, wide8, idx8, state,
-                           state + S_MAX_ABS, dev->nodes8);
-        BUILD_CHECK(hipGetLastError());
-        out->max_depth8 = depth8;
+    if (collapse_device<8>(d_nodes, n, state, limits.max_stack / 7, s, &wide8, &idx8, &depth8, &count8, &deep,
+                           error)) {
+        if (count8 <= limits.nodes8) {
+            BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&dev->nodes8), sizeof(BvhNode8Q) * count8));
+            dev->node8_count = count8;
+            const uint32_t grid8 = std::min<uint32_t>(blocks_for(count8), 2048);
+            hipLaunchKernelGGL(k_collapse_write8, dim3(grid8), dim3(BUILD_BLOCK), 0, nullptr, d_nodes, wide8, idx8,
+                               state, state + S_MAX_ABS, dev->nodes8);
+            BUILD_CHECK(hipGetLastError());
+            out->max_depth8 = depth8;
+        }
     } else if (!deep) {
         return false;
     }

@@ -276,20 +276,20 @@ struct Collapser8 {
 
 }  // namespace
 
-bool collapse_to_bvh8(const std::vector<BinaryNode>& bnodes, float max_abs, uint32_t max_stack, Bvh4* out) {
+bool collapse_to_bvh8(const std::vector<BinaryNode>& bnodes, float max_abs, const BvhLimits& limits, Bvh4* out) {
     Collapser8 col{bnodes, out->nodes8, 4e-6f * std::fmax(max_abs, 1e-3f)};
     out->nodes8.clear();
     out->nodes8.reserve(bnodes.size() / 4 + 1);
     col.collapse(0, 1);
     out->max_depth8 = col.max_depth;
-    if (7 * col.max_depth > max_stack) {  // too deep for the stack at 7 pushes per level: 4-wide only
+    if (7 * col.max_depth > limits.max_stack || out->nodes8.size() > limits.nodes8) {  // 4-wide only
         out->nodes8.clear();
         return false;
     }
     return true;
 }
 
-bool collapse_to_bvh4(const std::vector<BinaryNode>& bnodes, float max_abs, uint32_t max_stack, Bvh4* out,
+bool collapse_to_bvh4(const std::vector<BinaryNode>& bnodes, float max_abs, const BvhLimits& limits, Bvh4* out,
                       std::string* error) {
     // Boxes grow by an absolute margin proportional to the scene's extent so
     // the traversal's fused slab test stays conservative.
@@ -298,14 +298,18 @@ bool collapse_to_bvh4(const std::vector<BinaryNode>& bnodes, float max_abs, uint
     out->nodes.reserve(bnodes.size() / 2 + 1);
     col.collapse(0, 1);
     out->max_depth = col.max_depth;
-    if (3 * col.max_depth > max_stack) {
+    if (3 * col.max_depth > limits.max_stack) {
         *error = "BVH too deep for the traversal stack (depth " + std::to_string(col.max_depth) + ")";
+        return false;
+    }
+    if (out->nodes.size() > limits.nodes4) {
+        *error = "BVH of more nodes than the traversal addresses (" + std::to_string(out->nodes.size()) + ")";
         return false;
     }
     return true;
 }
 
-bool build_bvh4(const std::vector<WorldTriangle>& input, uint32_t max_stack, Bvh4* out, std::string* error) {
+bool build_bvh4(const std::vector<WorldTriangle>& input, const BvhLimits& limits, Bvh4* out, std::string* error) {
     const auto t0 = std::chrono::steady_clock::now();
     const uint32_t n = uint32_t(input.size());
     if (n == 0) {
@@ -342,10 +346,10 @@ bool build_bvh4(const std::vector<WorldTriangle>& input, uint32_t max_stack, Bvh
         Builder builder(prims, order, bnodes, rules);
         builder.build(0, 0, n, 0);
         bnodes.resize(builder.next.load());
-        return collapse_to_bvh4(bnodes, max_abs, max_stack, out, error);
+        return collapse_to_bvh4(bnodes, max_abs, limits, out, error);
     };
     if (!grow(BVH_RULES) && !grow(BVH_COARSE_RULES)) return false;
-    collapse_to_bvh8(bnodes, max_abs, max_stack, out);
+    collapse_to_bvh8(bnodes, max_abs, limits, out);
 
     out->tris.resize(n);
     for (uint32_t i = 0; i < n; ++i) {

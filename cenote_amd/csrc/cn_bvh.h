@@ -24,7 +24,7 @@ struct Bvh4 {
     uint32_t max_depth = 0;
     double build_seconds = 0.0;
     // The 8-wide collapse of the same binary tree over the same leaves,
-    // already quantized (empty when it would be too deep for the stack).
+    // already quantized (empty when it would be past the limits).
     std::vector<BvhNode8Q> nodes8;
     uint32_t max_depth8 = 0;
 };
@@ -38,26 +38,42 @@ struct BinaryNode {
 };
 static_assert(sizeof(BinaryNode) == 40, "device and host share this layout");
 
+// What a tree has to keep to: a 4-wide walk's stack takes three entries a
+// level and an 8-wide one's seven, and the walks address a node by a 32-bit
+// byte offset from the tree's base. LEAF_FIRST_MASK allows 2^27 triangles. By
+// BVH_RULES a triangle may be a leaf of its own, and the nodes may number two
+// thirds of them; by BVH_COARSE_RULES two triangles never part, a subtree of
+// two leaves holds at least three, and the nodes number at most 4/9 of them:
+// always fewer than nodes4.
+struct BvhLimits {
+    uint32_t max_stack;
+    uint32_t nodes4 = 1u << 26;
+    uint32_t nodes8 = 1u << 25;
+};
+static_assert(uint64_t(BvhLimits{}.nodes4) * sizeof(BvhNode4Q) <= uint64_t(1) << 32 &&
+                  uint64_t(BvhLimits{}.nodes8) * sizeof(BvhNode8Q) <= uint64_t(1) << 32,
+              "the last node starts below 2^32");
+
 // Binned-SAH binary build (32 bins on the three axes, leaves by BVH_RULES),
 // collapsed to 4-wide nodes by repeatedly opening the child of largest surface
-// area. A tree deeper than the traversal stack allows is grown again by
-// BVH_COARSE_RULES; returns false with a message when that is too deep too.
-bool build_bvh4(const std::vector<WorldTriangle>& input, uint32_t max_stack, Bvh4* out, std::string* error);
+// area. A tree past the limits is grown again by BVH_COARSE_RULES; returns
+// false with a message when that is past them too.
+bool build_bvh4(const std::vector<WorldTriangle>& input, const BvhLimits& limits, Bvh4* out, std::string* error);
 
 // The collapse step alone, from a binary tree rooted at node 0 (nodes may
 // be numbered in any order); max_abs is the scene's largest |coordinate|.
-bool collapse_to_bvh4(const std::vector<BinaryNode>& bnodes, float max_abs, uint32_t max_stack, Bvh4* out,
+bool collapse_to_bvh4(const std::vector<BinaryNode>& bnodes, float max_abs, const BvhLimits& limits, Bvh4* out,
                       std::string* error);
 
 // The 8-wide collapse of the same binary tree, by the same greedy rule up
 // to eight children, straight to BvhNode8Q; fills out->nodes8 and
-// max_depth8, or leaves nodes8 empty (returning false) when the tree is too
-// deep for `max_stack` at seven pushes per level.
-bool collapse_to_bvh8(const std::vector<BinaryNode>& bnodes, float max_abs, uint32_t max_stack, Bvh4* out);
+// max_depth8, or leaves nodes8 empty (returning false) when the tree is past
+// the limits.
+bool collapse_to_bvh8(const std::vector<BinaryNode>& bnodes, float max_abs, const BvhLimits& limits, Bvh4* out);
 
 // The device-resident outputs of the device builder: device allocations
 // the caller takes over (and frees with hipFree); nodes8 is null when the
-// 8-wide tree would be too deep for the stack.
+// 8-wide tree would be past the limits.
 struct DeviceBvh {
     BvhTriangle* tris = nullptr;
     BvhNode4Q* nodes = nullptr;
@@ -83,7 +99,7 @@ struct DeviceTriangles {
 // collapse to 4- and 8-wide
 // nodes and their quantization on the device, where the trees stay (`*dev`);
 // `out` receives the depths and the build time.
-bool build_bvh_device(const DeviceTriangles& input, uint32_t max_stack, Bvh4* out, DeviceBvh* dev,
+bool build_bvh_device(const DeviceTriangles& input, const BvhLimits& limits, Bvh4* out, DeviceBvh* dev,
                       std::string* error);
 
 // Rewrites, on the device, the flags word (v2.w) of every leaf-order

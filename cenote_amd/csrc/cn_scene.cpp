@@ -293,7 +293,7 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
     Bvh4 bvh;
     std::string error;
     if (host_built) {
-        if (!build_bvh4(world, STACK_MAX, &bvh, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
+        if (!build_bvh4(world, {STACK_MAX}, &bvh, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
         CN_HIP(scene->tris.upload(bvh.tris.data(), bvh.tris.size()));
         std::vector<BvhNode4Q> quantized(bvh.nodes.size());
         quantize_bvh4(bvh.nodes.data(), bvh.nodes.size(), quantized.data());
@@ -305,7 +305,7 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
         DeviceBvh dev;
         const DeviceTriangles input{scene->mesh_tris.ptr, scene->instances.ptr, tri_flags.data(), first.data(),
                                     desc->instance_count};
-        if (!build_bvh_device(input, STACK_MAX, &bvh, &dev, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
+        if (!build_bvh_device(input, {STACK_MAX}, &bvh, &dev, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
         scene->tris.adopt(dev.tris, triangle_count);
         scene->nodes.adopt(dev.nodes, dev.node_count);
         scene->full_nodes.adopt(dev.full, dev.node_count);

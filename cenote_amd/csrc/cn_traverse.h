@@ -227,9 +227,8 @@ __device__ __forceinline__ void order_pair(float& ka, uint32_t& ca, float& kb, u
 // keeps the test conservative.
 __device__ __forceinline__ uint32_t visit(const BvhNode4Q* __restrict__ nodes, uint32_t index, const Ray& r,
                                           float bound, Stack& st) {
-    // A 32-bit byte offset from the tree's base (a node index is below 2^26:
-    // leaves address at most 2^27 triangles, a node holds four children),
-    // so the fetch takes the base from scalar registers.
+    // A 32-bit byte offset from the tree's base (the builder keeps a tree
+    // below 2^26 nodes), so the fetch takes the base from scalar registers.
     const BvhNode4Q n =
         *reinterpret_cast<const BvhNode4Q*>(reinterpret_cast<const char*>(nodes) + index * uint32_t(sizeof(BvhNode4Q)));
     const float sx = n.step_x * r.ix;
@@ -272,7 +271,7 @@ __device__ __forceinline__ uint32_t visit(const BvhNode4Q* __restrict__ nodes, u
 // hit, visibility and transmittance do not depend on it.
 __device__ __forceinline__ uint32_t visit(const BvhNode8Q* __restrict__ nodes, uint32_t index, const Ray& r,
                                           float bound, Stack& st) {
-    // a 32-bit byte offset, as for the 4-wide nodes (8-wide indices are below 2^25)
+    // a 32-bit byte offset, as for the 4-wide nodes (fewer than 2^25 of these)
     const uint4* line =
         reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(nodes) + index * uint32_t(sizeof(BvhNode8Q)));
     const uint4 h = line[0];

@@ -22,19 +22,19 @@ def _library():
                     "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{source}", str(source / "cn_bvh.cpp"),
                     str(ROOT / "tests" / "native" / "bvh_host.cpp"), "-pthread", "-o", str(out)], check=True)
     lib = C.CDLL(str(out))
-    lib.bvh_host_build.argtypes = [C.c_void_p, C.c_uint32, C.c_uint32] + [C.POINTER(C.c_uint32)] * 4 + [
+    lib.bvh_host_build.argtypes = [C.c_void_p] + [C.c_uint32] * 4 + [C.POINTER(C.c_uint32)] * 4 + [
         C.c_char_p, C.c_size_t]
     return lib
 
 
-def build(corners, max_stack=STACK_MAX):
+def build(corners, max_stack=STACK_MAX, nodes4=1 << 26, nodes8=1 << 25):
     """The trees over (n, 3, 3) corners: their node counts and depths, and
     the refusal's text (empty when built)."""
     corners = np.ascontiguousarray(corners, np.float32)
     values = [C.c_uint32() for _ in range(4)]
     error = C.create_string_buffer(256)
-    _library().bvh_host_build(corners.ctypes.data_as(C.c_void_p), len(corners), max_stack,
-                              *[C.byref(v) for v in values], error, len(error))
+    _library().bvh_host_build(corners.ctypes.data_as(C.c_void_p), len(corners), max_stack, nodes4,
+                              nodes8, *[C.byref(v) for v in values], error, len(error))
     return dict(zip(("nodes4", "depth4", "nodes8", "depth8"), (v.value for v in values))), error.value.decode()
 
 
@@ -48,3 +48,9 @@ def chain(levels, cluster=6):
     at = np.concatenate([rng.uniform(0.9, 1.0, (n, 1, 1)), rng.uniform(0, 1, (n, 1, 2))], axis=2)
     shape = np.array([[0, 0, 0], [1e-3, 0, 0], [0, 1e-3, 1e-3]])
     return ((at + shape) * scale).astype(np.float32)
+
+
+def lattice(side):
+    """Small triangles far apart: every one of them a leaf of its own."""
+    at = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), axis=-1).reshape(-1, 1, 3)
+    return (at + np.array([[0, 0, 0], [1e-3, 0, 0], [0, 1e-3, 1e-3]])).astype(np.float32)

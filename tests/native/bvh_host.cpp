@@ -6,8 +6,9 @@
 
 #include "cn_bvh.h"
 
-extern "C" int bvh_host_build(const float* corners, uint32_t count, uint32_t max_stack, uint32_t* nodes4,
-                              uint32_t* depth4, uint32_t* nodes8, uint32_t* depth8, char* error, size_t capacity) {
+extern "C" int bvh_host_build(const float* corners, uint32_t count, uint32_t max_stack, uint32_t most4,
+                              uint32_t most8, uint32_t* nodes4, uint32_t* depth4, uint32_t* nodes8, uint32_t* depth8,
+                              char* error, size_t capacity) {
     std::vector<cn::WorldTriangle> input(count);
     for (uint32_t i = 0; i < count; ++i) {
         const float* p = corners + 9 * size_t(i);
@@ -15,7 +16,7 @@ extern "C" int bvh_host_build(const float* corners, uint32_t count, uint32_t max
     }
     cn::Bvh4 out;
     std::string message;
-    const bool ok = cn::build_bvh4(input, max_stack, &out, &message);
+    const bool ok = cn::build_bvh4(input, {max_stack, most4, most8}, &out, &message);
     *nodes4 = uint32_t(out.nodes.size());
     *depth4 = out.max_depth;
     *nodes8 = uint32_t(out.nodes8.size());
