@@ -153,8 +153,9 @@ static int read_pieces(int device, Readback& rb, const ReadArray* arrays, int n)
             failed.store(int(e));
         }
     };
-    // The calling thread is worker 0; a thread that cannot be had leaves its
-    // share to the others.
+    // The calling thread is worker 0; a thread that cannot be had (the system's
+    // limit, or no memory for its state) leaves its share to the others. Nothing
+    // may leave this scope before they are joined.
     const int workers = int(std::min<size_t>(Readback::WORKERS, pieces.size() / 2));
     std::vector<std::thread> threads;
     threads.reserve(workers);
@@ -162,6 +163,8 @@ static int read_pieces(int device, Readback& rb, const ReadArray* arrays, int n)
         try {
             threads.emplace_back(work, w);
         } catch (const std::system_error&) {
+            break;
+        } catch (const std::bad_alloc&) {
             break;
         }
     }
