@@ -6,8 +6,9 @@
 // fmaf appears only where the reference kernels call fma. dot products
 // accumulate x, y, z left to right; normalize(v) = v * (1/sqrt(v.v));
 // lerp(x, y, a) = x*(1-a) + y*a (the SPIR-V FMix definition the reference's
-// `lerp` lowers to). Division and sqrt are IEEE correctly rounded (HIP's
-// default for f32).
+// `lerp` lowers to). The operators / and sqrtf are IEEE correctly rounded
+// (HIP's default for f32); rcp_n, div_n and sqrt_n below are within their
+// stated ranges.
 #pragma once
 
 #include <stdint.h>
@@ -69,17 +70,21 @@ __host__ __device__ __forceinline__ float4 F4(v3 v, float w) { return make_float
 // kernel's code. Without the scaling, one Newton step on v_rcp_f32 (Markstein:
 // a correctly rounded reciprocal and one residual correction give the
 // correctly rounded quotient) and the fixup for zeros, infinities and NaN:
-//  * rcp_n: every float of exponent 2^-126 to 2^125 (all of them tried on the
-//    device);
-//  * div_n: a divisor in that range and a dividend and quotient of at least
-//    2^-100 (every mantissa's reciprocal is exact; 2^35 random pairs within
-//    2^+-20 and 2^32 within 2^+-60 tried): smaller ones may lose a last bit;
+//  * rcp_n: every float of magnitude 2^-126 to 2^125 (all of them tried);
+//  * div_n: a divisor in that range, a dividend and a quotient of magnitude
+//    2^-100 to 2^126 (2^32 random pairs tried, among them the ends of the
+//    mantissas; every mantissa's reciprocal is exact);
 //  * sqrt_n: 0, infinity and every float from 2^-101 (all tried).
-// They stand where the operands' range is known: unit vectors, roughnesses,
-// weights, angles. Lengths, areas and densities whose scale the scene sets
-// keep the operators. With them (and one sincosf for a sine and a cosine) the
-// shading kernel's code went from 68 to 45 KB and its time per frame from 8.28
-// to 7.9 ms on the chart and 12.6 to 12.2 on the 2M-triangle scene.
+// Outside: smaller dividends and quotients may lose a last bit; a divisor above
+// 2^126 has a reciprocal that v_rcp_f32 flushes, and a quotient past the
+// largest float or one by a subnormal number comes out NaN, not infinite; the
+// root of a subnormal number may come out NaN. So they stand where the
+// operands' range is known: unit vectors, roughnesses, weights, colours, angles.
+// Lengths, areas, densities and indices of refraction, whose scale the scene
+// sets, keep the operators. With them (and one sincosf for a sine and a
+// cosine) the shading kernel's code went from 68 to 45 KB and its time per
+// frame from 8.28 to 7.9 ms on the chart and 12.6 to 12.2 on the 2M-triangle
+// scene.
 __device__ __forceinline__ float rcp_step(float b) {
     const float y = __builtin_amdgcn_rcpf(b);
     return fmaf(fmaf(-b, y, 1.0f), y, y);

@@ -109,7 +109,10 @@ __device__ __forceinline__ float tab3(const float* t, uint32_t off, float x, flo
     return lerpf(tab2(t, off + 256u * i, 16, 16, x, y), tab2(t, off + 256u * j, 16, 16, x, y), fz - float(i));
 }
 
-__device__ __forceinline__ float ior_remap(float eta) { return sqrt_n(div_n(fabsf(eta - 1.0f), eta + 1.0f)); }
+// An index of refraction comes from the scene, at any scale (cn_math.h): the
+// quotients of one are the operators' wherever it is not the closure's own
+// (0, 2^-25 to 2^25, or infinite).
+__device__ __forceinline__ float ior_remap(float eta) { return sqrt_n(fabsf(eta - 1.0f) / (eta + 1.0f)); }
 
 // --- EON diffuse (openpbr.slang:134-175) ----------------------------------------
 
@@ -173,22 +176,24 @@ __device__ __forceinline__ v3 fresnel_schlick(v3 f0, float cosine) {
     return f0 + (((1.0f - f0) * m2) * m2) * m;
 }
 
+template <bool SCENE_IOR = false>  // not the closure's own
 __device__ __forceinline__ float fresnel_dielectric(float eta, float cosine) {
+    const auto quotient = [](float a, float b) { return SCENE_IOR ? a / b : div_n(a, b); };
     const float mu = fabsf(cosine);
     const float sin2 = 1.0f - mu * mu;
-    const float cos2t = 1.0f - div_n(sin2, eta * eta);
+    const float cos2t = 1.0f - quotient(sin2, eta * eta);
     if (cos2t < 0.0f) return 1.0f;
     const float t0 = sqrt_n(cos2t);
     const float t1 = eta * t0;
     const float t2 = eta * mu;
-    const float rs = div_n(mu - t1, mu + t1);
-    const float rp = div_n(t0 - t2, t0 + t2);
+    const float rs = quotient(mu - t1, mu + t1);
+    const float rp = quotient(t0 - t2, t0 + t2);
     return (rs * rs + rp * rp) / 2.0f;
 }
 
 __device__ __forceinline__ float fresnel_dielectric_avg(float eta) {
     if (eta < 1.0f) return 0.997118f + eta * (0.1014f - eta * (0.965241f + eta * 0.130607f));
-    return div_n(eta - 1.0f, 4.08567f + 1.00071f * eta);
+    return (eta - 1.0f) / (4.08567f + 1.00071f * eta);
 }
 
 __device__ __forceinline__ v3 fresnel_ms(v3 fss, float eAvg) {
@@ -222,16 +227,17 @@ __device__ __forceinline__ v3 reflection_scale(const float* t, float rough, floa
 }
 
 // openpbr.slang:357-363
+template <bool SCENE_IOR = false>
 __device__ __forceinline__ float dielectric_albedo(const float* t, float rough, float mu, float eta) {
-    if (eta < 1.0f) return fresnel_dielectric(eta, mu);
+    if (eta < 1.0f) return fresnel_dielectric<SCENE_IOR>(eta, mu);
     return tab3(t, T_DIELECTRIC_E, rough, mu, ior_remap(eta));
 }
 
 // openpbr.slang:371-384
 __device__ __forceinline__ v3 coat_darkening(const Mat& m, float rough, float mu, float baseFresnel) {
     const float fssCoat = fresnel_dielectric_avg(m.coatIor);
-    const float kRough = 1.0f - div_n(1.0f - fssCoat, m.coatIor * m.coatIor);
-    const float kSmooth = fresnel_dielectric(m.coatIor, mu);
+    const float kRough = 1.0f - (1.0f - fssCoat) / (m.coatIor * m.coatIor);
+    const float kSmooth = fresnel_dielectric<true>(m.coatIor, mu);
     const float roughDiffuse = lerpf(1.0f, rough, saturate(m.specularWeight * baseFresnel));
     const float baseRough = lerpf(roughDiffuse, rough, m.metalness);
     const float k = lerpf(kSmooth, kRough, baseRough);
@@ -261,10 +267,10 @@ __device__ inline Closure resolve_closure(const float* t, const Mat& m, v3 wo, b
 
     float etaS = fmaxf(m.specularIor, 1e-4f);
     if (coated) {
-        const float etaBc = m.coatIor > etaS ? div_n(m.coatIor, etaS) : div_n(etaS, m.coatIor);
+        const float etaBc = m.coatIor > etaS ? m.coatIor / etaS : etaS / m.coatIor;
         etaS = lerpf(etaS, etaBc, m.coatWeight);
     }
-    const float f0 = div_n((etaS - 1.0f) * (etaS - 1.0f), (etaS + 1.0f) * (etaS + 1.0f));
+    const float f0 = (etaS - 1.0f) * (etaS - 1.0f) / ((etaS + 1.0f) * (etaS + 1.0f));
     const float weight = clampf(m.specularWeight, 0.0f, f0 > 1e-6f ? rcp_n(f0) : 0.0f);
     const float epsilon = signf(etaS - 1.0f) * sqrtf(weight * f0);
     float eta = div_n(1.0f + epsilon, fmaxf(1e-3f, 1.0f - epsilon));
@@ -291,7 +297,7 @@ __device__ inline Closure resolve_closure(const float* t, const Mat& m, v3 wo, b
     c.coatScale = 1.0f;
     v3 coatAtten = S3(1.0f);
     if (coated) {
-        c.coatE = dielectric_albedo(t, coatRough, mu, m.coatIor);
+        c.coatE = dielectric_albedo<true>(t, coatRough, mu, m.coatIor);
         const float fssCoat = fresnel_dielectric_avg(m.coatIor);
         c.coatScale = reflection_scale(t, coatRough, mu, S3(fssCoat)).x;
         coatAtten = vlerp(S3(1.0f), m.coatColor * (1.0f - c.coatE), m.coatWeight) * coat_darkening(m, rough, mu, f0);
@@ -475,7 +481,7 @@ __device__ inline v3 eval_bsdf(const Closure& c, v3 wi, v3 wo) {
     }
     const v3 h = normalize(wi + wo);
     if (m.coatWeight > 0.0f && !c.exiting) {
-        const float coatF = fresnel_dielectric(m.coatIor, dot(h, wo));
+        const float coatF = fresnel_dielectric<true>(m.coatIor, dot(h, wo));
         result = result + S3(c.fuzzAtten * m.coatWeight * coatF * c.coatScale * reflection_core(c.coatAlpha, wi, wo, h));
     }
     v3 base = S3(0.0f);
@@ -612,7 +618,7 @@ __device__ inline BsdfEval eval_with_pdf(const Closure& c, v3 wi, v3 wo) {
     v3 result = S3(0.0f);
     if (fuzzF) result = result + div_n(((m.fuzzWeight * m.fuzzColor) * c.fuzzR) * density, wi.z);
     if (coatF) {
-        const float coatFresnel = fresnel_dielectric(m.coatIor, cosVH);
+        const float coatFresnel = fresnel_dielectric<true>(m.coatIor, cosVH);
         const float core = div_n(coatD * coatG1o * smith_g1(c.coatAlpha, wi.z), 4.0f * wo.z * wi.z);
         result = result + S3(c.fuzzAtten * m.coatWeight * coatFresnel * c.coatScale * core);
     }
@@ -820,7 +826,7 @@ __device__ __forceinline__ float env_pdf(const SceneView& s, v3 d) {
     const f2 uv = uv_from_direction(d);
     const uint32_t col = min(uint32_t(uv.x * float(s.env_width)), s.env_width - 1);
     const uint32_t row = min(uint32_t(uv.y * float(s.env_height)), s.env_height - 1);
-    return div_n(s.env_pdfs[row * s.env_width + col], 2.0f * PI_K * PI_K * sinTheta);
+    return s.env_pdfs[row * s.env_width + col] / (2.0f * PI_K * PI_K * sinTheta);
 }
 
 // lights.slang:42-44
