@@ -1093,8 +1093,9 @@ __device__ void quantize_axis(const float* lo, const float* hi, int count, float
     *exps_byte = uint32_t(e + 127);
 }
 
-// Every 4-wide node at its preorder index: the full-precision record (the
-// host collapse's set_child with the same padding) and its quantized form.
+// Every 4-wide node at its preorder index: its quantized form, and where
+// `full` is given the full-precision record (the host collapse's set_child
+// with the same padding).
 __global__ __launch_bounds__(BUILD_BLOCK) void k_collapse_write4(const BinaryNode* __restrict__ nodes,
                                                                  const WideTmp<4>* __restrict__ wide,
                                                                  const uint32_t* __restrict__ indices,
@@ -1128,7 +1129,7 @@ __global__ __launch_bounds__(BUILD_BLOCK) void k_collapse_write4(const BinaryNod
             ch[k] = child_ref(nodes, w.kid[k], w.kid_wide[k], indices);
         }
         n.meta = make_uint4(w.depth, 0, 0, 0);
-        full[w.index] = n;
+        if (full) full[w.index] = n;
         BvhNode4Q q{};
         const float* los[3] = {lx, ly, lz};
         const float* his[3] = {hx, hy, hz};
@@ -1309,8 +1310,8 @@ bool collapse_device(const BinaryNode* d_nodes, uint32_t n, uint32_t* state, uin
 
 }  // namespace
 
-bool build_bvh_device(const DeviceTriangles& input, const BvhLimits& limits, Bvh4* out, DeviceBvh* dev,
-                      std::string* error) {
+bool build_bvh_device(const DeviceTriangles& input, const BvhLimits& limits, bool full_nodes, Bvh4* out,
+                      DeviceBvh* dev, std::string* error) {
     const auto t0 = std::chrono::steady_clock::now();
     *dev = DeviceBvh{};
     // The outputs are freed again unless the build finishes.
@@ -1319,8 +1320,7 @@ bool build_bvh_device(const DeviceTriangles& input, const BvhLimits& limits, Bvh
         bool keep = false;
         ~Outputs() {
             if (keep) return;
-            for (void* p : {static_cast<void*>(d->tris), static_cast<void*>(d->nodes), static_cast<void*>(d->nodes8),
-                            static_cast<void*>(d->full)})
+            for (void* p : {static_cast<void*>(d->tris), static_cast<void*>(d->nodes), static_cast<void*>(d->nodes8)})
                 if (p) (void)hipFree(p);
             *d = DeviceBvh{};
         }
@@ -1487,13 +1487,21 @@ bool build_bvh_device(const DeviceTriangles& input, const BvhLimits& limits, Bvh
         *error = "BVH of more nodes than the traversal addresses (" + std::to_string(count4) + ")";
         return false;
     }
-    BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&dev->full), sizeof(BvhNode4) * count4));
+    BvhNode4* full = full_nodes ? s.get<BvhNode4>(count4) : nullptr;
+    if (full_nodes && !full) {
+        *error = "device BVH build: out of device memory";
+        return false;
+    }
     BUILD_CHECK(hipMalloc(reinterpret_cast<void**>(&dev->nodes), sizeof(BvhNode4Q) * count4));
     dev->node_count = count4;
     const uint32_t grid4 = std::min<uint32_t>(blocks_for(count4), 2048);
     hipLaunchKernelGGL(k_collapse_write4, dim3(grid4), dim3(BUILD_BLOCK), 0, nullptr, d_nodes, wide4, idx4, state,
-                       state + S_MAX_ABS, dev->full, dev->nodes);
+                       state + S_MAX_ABS, full, dev->nodes);
     BUILD_CHECK(hipGetLastError());
+    if (full_nodes) {
+        out->nodes.resize(count4);
+        BUILD_CHECK(hipMemcpy(out->nodes.data(), full, sizeof(BvhNode4) * count4, hipMemcpyDeviceToHost));
+    }
     out->max_depth = depth4;
 
     WideTmp<8>* wide8 = nullptr;

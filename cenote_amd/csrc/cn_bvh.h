@@ -78,7 +78,6 @@ struct DeviceBvh {
     BvhTriangle* tris = nullptr;
     BvhNode4Q* nodes = nullptr;
     BvhNode8Q* nodes8 = nullptr;
-    BvhNode4* full = nullptr;  // the full-precision nodes, for read-back
     uint32_t node_count = 0, node8_count = 0;
 };
 
@@ -96,11 +95,12 @@ struct DeviceTriangles {
 // The same trees built entirely on the device (cn_build.hip): top levels by
 // device-wide binning with every split decided on the device, subtrees of
 // <= 2048 triangles by one workgroup each and of <= 64 by one wave each, the
-// collapse to 4- and 8-wide
-// nodes and their quantization on the device, where the trees stay (`*dev`);
-// `out` receives the depths and the build time.
-bool build_bvh_device(const DeviceTriangles& input, const BvhLimits& limits, Bvh4* out, DeviceBvh* dev,
-                      std::string* error);
+// collapse to 4- and 8-wide nodes and their quantization on the device, where
+// the trees stay (`*dev`); `out` receives the depths and the build time, and
+// with `full_nodes` the full-precision 4-wide nodes, which no walk reads.
+// Building the same triangles again gives the same records.
+bool build_bvh_device(const DeviceTriangles& input, const BvhLimits& limits, bool full_nodes, Bvh4* out,
+                      DeviceBvh* dev, std::string* error);
 
 // Rewrites, on the device, the flags word (v2.w) of every leaf-order
 // triangle from its instance's entry in `instance_flags` (host array of

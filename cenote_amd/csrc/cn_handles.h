@@ -111,7 +111,7 @@ struct cn_scene {
     cn_camera camera{};
     cn::DevBuf<cn::BvhNode4Q> nodes;        // what the traversal reads
     cn::DevBuf<cn::BvhNode4P> pnodes;       // the same nodes decoded for camera-ray packets
-    cn::DevBuf<cn::BvhNode4> full_nodes;    // the full-precision tree (cn_scene_bvh)
+    std::vector<cn::BvhNode4> host_nodes;   // the full-precision tree of the host builder (cn_scene_bvh)
     cn::DevBuf<cn::BvhNode8Q> nodes8;       // the 8-wide tree over the same leaves (may be empty)
     cn::DevBuf<cn::BvhTriangle> tris;
     cn::DevBuf<cn::InstanceRecord> instances;

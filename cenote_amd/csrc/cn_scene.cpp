@@ -299,16 +299,15 @@ int prep_scene(cn_context* ctx, const cn_scene_desc* desc, cn_scene* scene) {
         quantize_bvh4(bvh.nodes.data(), bvh.nodes.size(), quantized.data());
         CN_HIP(scene->nodes.upload(quantized.data(), quantized.size()));
         if (!bvh.nodes8.empty()) CN_HIP(scene->nodes8.upload(bvh.nodes8.data(), bvh.nodes8.size()));
-        CN_HIP(scene->full_nodes.upload(bvh.nodes.data(), bvh.nodes.size()));
+        scene->host_nodes = std::move(bvh.nodes);
     } else {
         // Built, collapsed and quantized on the device, and kept there.
         DeviceBvh dev;
         const DeviceTriangles input{scene->mesh_tris.ptr, scene->instances.ptr, tri_flags.data(), first.data(),
                                     desc->instance_count};
-        if (!build_bvh_device(input, {STACK_MAX}, &bvh, &dev, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
+        if (!build_bvh_device(input, {STACK_MAX}, false, &bvh, &dev, &error)) return fail(CN_E_SCENE, "%s", error.c_str());
         scene->tris.adopt(dev.tris, triangle_count);
         scene->nodes.adopt(dev.nodes, dev.node_count);
-        scene->full_nodes.adopt(dev.full, dev.node_count);
         if (dev.nodes8) scene->nodes8.adopt(dev.nodes8, dev.node8_count);
     }
     CN_HIP(scene->pnodes.alloc(scene->nodes.count));
@@ -363,6 +362,36 @@ bool same_geometry(const cn_scene* scene, const cn_scene_desc* desc) {
         }
     }
     return true;
+}
+
+// The full-precision 4-wide nodes into host memory. The device builder's are
+// grown again from the resident triangles instead of being kept: 128 bytes a
+// node (104 MB of the 2M-triangle scene's memory) that nothing else reads.
+int copy_full_nodes(const cn_scene* scene, void* out) {
+    const std::vector<BvhNode4>* nodes = &scene->host_nodes;
+    Bvh4 bvh;
+    if (scene->info.bvh_builder == CN_BVH_DEVICE) {
+        const uint32_t count = scene->info.instance_count;
+        const std::vector<uint32_t> flags(count, 0u);  // no node holds them
+        std::vector<size_t> first(size_t(count) + 1, 0);
+        for (uint32_t i = 0; i < count; ++i)
+            first[i + 1] = first[i] + scene->host_mesh_shape[2 * size_t(scene->host_instance_mesh[i]) + 1];
+        const DeviceTriangles input{scene->mesh_tris.ptr, scene->instances.ptr, flags.data(), first.data(), count};
+        DeviceBvh dev;
+        std::string error;
+        if (!build_bvh_device(input, {STACK_MAX}, true, &bvh, &dev, &error))
+            return fail(CN_E_SCENE, "%s", error.c_str());
+        DevBuf<BvhTriangle> tris;
+        DevBuf<BvhNode4Q> quantized;
+        DevBuf<BvhNode8Q> quantized8;
+        tris.adopt(dev.tris, scene->tris.count);
+        quantized.adopt(dev.nodes, dev.node_count);
+        if (dev.nodes8) quantized8.adopt(dev.nodes8, dev.node8_count);
+        nodes = &bvh.nodes;
+    }
+    if (nodes->size() != scene->nodes.count) return fail(CN_E_DEVICE_FAULT, "the resident tree did not grow again");
+    std::memcpy(out, nodes->data(), nodes->size() * sizeof(BvhNode4));
+    return CN_OK;
 }
 
 }  // namespace
@@ -500,11 +529,11 @@ int cn_scene_bvh(cn_scene* scene, void* nodes, uint32_t node_capacity, uint32_t*
                  uint32_t triangle_capacity, uint32_t* triangle_count) {
     if (!scene) return fail(CN_E_INVALID, "cn_scene_bvh: null scene");
     CN_HIP(hipSetDevice(scene->ctx->device));
-    if (node_count) *node_count = uint32_t(scene->full_nodes.count);
+    if (node_count) *node_count = uint32_t(scene->nodes.count);
     if (triangle_count) *triangle_count = uint32_t(scene->tris.count);
     if (nodes) {
-        if (node_capacity < scene->full_nodes.count) return fail(CN_E_INVALID, "node buffer too small");
-        CN_HIP(hipMemcpy(nodes, scene->full_nodes.ptr, scene->full_nodes.count * sizeof(BvhNode4), hipMemcpyDeviceToHost));
+        if (node_capacity < scene->nodes.count) return fail(CN_E_INVALID, "node buffer too small");
+        if (int e = copy_full_nodes(scene, nodes)) return e;
     }
     if (triangles) {
         if (triangle_capacity < scene->tris.count) return fail(CN_E_INVALID, "triangle buffer too small");

@@ -305,7 +305,8 @@ int cn_scene_info_get(cn_scene* scene, cn_scene_info* info);
  * child slab bounds, child refs, meta) and the 48-byte leaf-order triangles
  * the traversal reads (either output may be NULL; *count gets the record
  * count). The traversal reads each node quantized to 64 bytes, as
- * cn_bvh_quantize computes it. */
+ * cn_bvh_quantize computes it; the full-precision nodes of a device-built
+ * scene are not resident, so asking for them builds its tree once more. */
 int cn_scene_bvh(cn_scene* scene, void* nodes, uint32_t node_capacity, uint32_t* node_count, void* triangles,
                  uint32_t triangle_capacity, uint32_t* triangle_count);
 /* The 8-wide traversal nodes (128 bytes each: a grid origin and three
