@@ -131,10 +131,32 @@ def waves_per_frame(width, height, spp, capacity):
     return -(-spp // per)
 
 
+def ranges_per_wave(width, height, capacity):
+    """Pool-sized ranges of paths that a wave walks: one, unless a single sample overfills the pool."""
+    return max(1, -(-width * height // capacity))
+
+
 def tail_split(depth, tail):
     """The bounce the tail launch takes over after (its trace is the last
     wavefront trace), or `depth` when every bounce runs as stages."""
     return tail if 0 < tail < depth else depth
+
+
+# A bounce of no more rays is left to the tail launch ahead of its own bounce
+# (cn_stages.hip), and a range of no more paths launches it right after bounce
+# 1's trace (cn_launch.h).
+TAIL_PATHS = 16384
+TAIL_AT_ONCE = 8192
+
+
+def tail_start(rays, tail, ranges=1):
+    """The bounce from which the tail launch carries the paths of a wave with
+    `rays` by bounce (their number when no tail runs). The rays of several
+    ranges are taken as equal shares."""
+    t = tail_split(len(rays), tail)
+    if t == len(rays):
+        return t
+    return next((b for b in range(1, t) if rays[b] <= TAIL_PATHS * ranges), t)
 
 
 def timed_launches(name, steps, capacity, tail=0):
@@ -143,12 +165,14 @@ def timed_launches(name, steps, capacity, tail=0):
 
     cfg = workloads.CONFIGS[name]
     waves = waves_per_frame(cfg["width"], cfg["height"], cfg["spp"], capacity) * steps
+    ranges = waves * ranges_per_wave(cfg["width"], cfg["height"], capacity)
     depth = cfg["max_bounces"]
     t = tail_split(depth, tail)
-    traced = waves * min(depth, t + 1)
+    if t < depth and min(capacity, cfg["width"] * cfg["height"] * cfg["spp"]) <= TAIL_AT_ONCE:
+        t = 1
     # bounce 0's misses are shaded by its trace launch
-    return {"raygen": waves, "trace": traced, "shade_miss": waves * max(0, t - 1), "shade_surface": waves * t,
-            "accumulate": waves, "tail": waves if t < depth else 0}
+    return {"raygen": ranges, "trace": ranges * min(depth, t + 1), "shade_miss": ranges * max(0, t - 1),
+            "shade_surface": ranges * t, "accumulate": waves, "tail": ranges if t < depth else 0}
 
 
 def shape_key(name, capacity, width=4, tail=0):
@@ -173,40 +197,47 @@ def load_traffic(key):
     return entry if isinstance(entry, dict) else None
 
 
-def algorithmic_bytes(counts, by_bounce, info, pixels, aov, width=4, tail=0, counter_lines=0):
+def algorithmic_bytes(waves, info, pixels, aov, width=4, tail=0, counter_lines=0, ranges=1):
     """Per-kernel algorithmic bytes of the counted waves, bounce by bounce; a
     node fetch counts its record size (64 bytes 4-wide, 128 bytes 8-wide).
-    With a tail after bounce t, trace holds bounces 0..t (and the camera
-    paths' generation and bounce 0's miss shading, which its bounce-0 launch
-    does: the reference's raygen stage, 72 bytes per path), shade_miss
-    bounces 1..t-1, shade_surface bounces 0..t-1, and the tail kernel every
-    later trace and all shading from bounce t on. raygen itself only resets
-    the range's queue counters (128 bytes a counter line). `by_bounce[b]` = ray nodes, ray triangles,
-    shadow nodes, shadow triangles of bounce b's trace launch (whose shadow
-    rays are bounce b-1's connections)."""
+    With a tail from bounce t of a wave on (tail_start), trace holds bounces
+    0..t (and the camera paths' generation and bounce 0's miss shading, which
+    its bounce-0 launch does: the reference's raygen stage, 72 bytes per path),
+    shade_miss bounces 1..t-1, shade_surface bounces 0..t-1, and the tail kernel
+    every later trace and all shading from bounce t on. raygen itself only
+    resets the range's queue counters (128 bytes a counter line). `waves` holds
+    each wave's stage counts and its traversal's: `by_bounce[b]` = ray nodes,
+    ray triangles, shadow nodes, shadow triangles of bounce b's trace launch
+    (whose shadow rays are bounce b-1's connections)."""
     node = 128 if width == 8 else info.bvh_node_bytes
     tri = info.bvh_triangle_bytes
-    depth = len(counts["rays"])
-    traced, surface, miss = [], [], []
-    for b in range(depth):
-        rn, rt, sn, st = (int(v) for v in by_bounce[b])
-        connections = int(counts["shadows"][b - 1]) if b > 0 else 0
-        # intersect fused with the previous bounce's trace_shadow
-        traced.append(BYTES["ray"] * int(counts["rays"][b]) + node * rn + tri * rt
-                      + BYTES["shadow"] * connections + node * sn + tri * st)
-        surface.append(BYTES["hit"] * int(counts["hits"][b]))
-        miss.append(BYTES["miss"] * int(counts["misses"][b]))
-    t = tail_split(depth, tail)
     out = {
         "raygen": counter_lines * 128,
         "accumulate": pixels * (BYTES["camera_path_aov"] if aov else 48),
-        "trace": sum(traced[: t + 1]) + miss[0] + pixels * 72,
-        "shade_surface": sum(surface[:t]),
-        "shade_miss": sum(miss[1:t]),
+        "trace": pixels * 72,
+        "shade_surface": 0,
+        "shade_miss": 0,
     }
-    if t < depth:
-        out["tail"] = sum(traced[t + 1:]) + sum(surface[t:]) + sum(miss[t:])
-    totals = {k: int(counts[k].sum()) for k in ("rays", "hits", "misses", "shadows")}
+    totals = dict.fromkeys(("rays", "hits", "misses", "shadows"), 0)
+    for counts, by_bounce in waves:
+        depth = len(counts["rays"])
+        traced, surface, miss = [], [], []
+        for b in range(depth):
+            rn, rt, sn, st = (int(v) for v in by_bounce[b])
+            connections = int(counts["shadows"][b - 1]) if b > 0 else 0
+            # intersect fused with the previous bounce's trace_shadow
+            traced.append(BYTES["ray"] * int(counts["rays"][b]) + node * rn + tri * rt
+                          + BYTES["shadow"] * connections + node * sn + tri * st)
+            surface.append(BYTES["hit"] * int(counts["hits"][b]))
+            miss.append(BYTES["miss"] * int(counts["misses"][b]))
+        t = tail_start(counts["rays"], tail, ranges)
+        out["trace"] += sum(traced[: t + 1]) + miss[0]
+        out["shade_surface"] += sum(surface[:t])
+        out["shade_miss"] += sum(miss[1:t])
+        if tail_split(depth, tail) < depth:
+            out["tail"] = out.get("tail", 0) + sum(traced[t + 1:]) + sum(surface[t:]) + sum(miss[t:])
+        for k in totals:
+            totals[k] += int(counts[k].sum())
     return out, totals
 
 
@@ -244,17 +275,17 @@ def measure_plain(ctx, name, steps, warmup, capacity=0, data=None, cpu=False, bv
     # Counting pass: one frame (every frame traces the same samples), with
     # traversal counters on, for the algorithmic-bytes model.
     renderer.set_counters(True)
-    counts = None
+    waves = []  # each wave's counts, and its traversal's by bounce
     film.reset()
-    done = 0
+    done, before = 0, 0
     while done < spp:
         n = min(per_wave, spp - done)
         renderer.accumulate(scene, film, count=n)
-        c = renderer.wave_counts()
-        counts = c if counts is None else {k: counts[k] + c[k] for k in c}
+        by_bounce = renderer.traversal_counts_by_bounce()
+        waves.append((renderer.wave_counts(), by_bounce - before))
+        before = by_bounce
         done += n
     traversal = renderer.traversal_counts()
-    by_bounce = renderer.traversal_counts_by_bounce()
     renderer.set_counters(False)
     tail = renderer.shape["tail_bounce"]
 
@@ -274,9 +305,11 @@ def measure_plain(ctx, name, steps, warmup, capacity=0, data=None, cpu=False, bv
     renderer.set_profiling(False)
 
     # the ranges' counter lines: 4 queues x 8 sub-queues per bounce, plus a spare
-    # bounce, then the tail launch's 8 item counters
-    lines = ((depth + 1) * 4 * 8 + 8 + depth * 8) * waves_per_frame(width, height, spp, renderer.capacity)
-    frame_bytes, totals = algorithmic_bytes(counts, by_bounce, info, pixels * spp, aov, walked, tail, lines)
+    # bounce, then 8 item counters of the tail launch and 8 chunk counters of each
+    # bounce's trace launch
+    ranges = ranges_per_wave(width, height, renderer.capacity)
+    lines = ((depth + 1) * 4 * 8 + 8 + depth * 8) * ranges * waves_per_frame(width, height, spp, renderer.capacity)
+    frame_bytes, totals = algorithmic_bytes(waves, info, pixels * spp, aov, walked, tail, lines, ranges)
     value = pixels * spp * steps / elapsed / 1e6
     grays = (totals["rays"] + totals["shadows"]) * steps / elapsed / 1e9
     kernel_ms = {k: round(v[0] / steps, 4) for k, v in times.items()}
@@ -289,7 +322,8 @@ def measure_plain(ctx, name, steps, warmup, capacity=0, data=None, cpu=False, bv
     key = shape_key(name, renderer.capacity, walked, tail)
     measured = load_traffic(key)
     traffic = None if measured is None else measured.get(dominant)
-    hit_share = totals["hits"] and float(counts["hits"][0]) / float(counts["hits"][0] + counts["misses"][0])
+    camera_hits = sum(int(c["hits"][0]) for c, _ in waves)
+    hit_share = totals["hits"] and camera_hits / float(camera_hits + sum(int(c["misses"][0]) for c, _ in waves))
     log(f"{name}: per frame rays {totals['rays']}, hits {totals['hits']}, misses {totals['misses']}, "
         f"shadows {totals['shadows']}; camera-ray hit share {hit_share:.3f}; "
         f"nodes/ray {traversal['ray_nodes'] / max(1, totals['rays']):.1f}, "
