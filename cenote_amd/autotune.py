@@ -1,6 +1,6 @@
 """Launch-shape autotuner for the wavefront stages.
 
-The stage kernels' launch shape — the persistent trace grid, the
+The stage kernels' launch shape — the trace grid, the
 shade_surface workgroup variant (1024/512/256 lanes with the BSDF tables in
 LDS, or 256 lanes reading them through the caches), the shading grid caps
 the BVH width the traversal walks and the bounce from which one tail launch
@@ -34,7 +34,9 @@ SHADE_VARIANTS = {
 
 def candidate_shapes(compute_units: int, trace_per_cu=(16, 32, 64), variants=tuple(SHADE_VARIANTS), widths=(4, 8),
                      tails=(_abi.DEFAULT_TAIL_BOUNCE,)):
-    """The default search grid: trace workgroups per CU x shade variants x
+    """The default search grid: trace workgroups per CU (of bounce 0's launch;
+    later bounces run no more than the chip holds at once, 8 or 7 per CU, so
+    values above that differ in bounce 0 alone) x shade variants x
     BVH width (the 4- or 8-wide tree a scene carries) x tail bounce (0: the
     wavefront stages throughout; by default only the library's own), with
     each shade variant's grid capped at 2048 lanes per CU (4096 for the

@@ -32,7 +32,8 @@ inline uint32_t shade_block(uint32_t variant) {
 // Grid sizes: the traversal kernels run a fixed, chip-filling grid and
 // walk their queue; the shading kernels are capped likewise.
 struct LaunchShape {
-    uint32_t trace_blocks;   // blocks of 256 lanes for trace
+    uint32_t trace_blocks;   // most blocks of 256 lanes for trace and the tail (bounces from 1 on run no
+                             // more than the chip holds at once, 8 or 7 per CU, the tail 3 per CU)
     uint32_t shade_variant;  // a ShadeVariant
     uint32_t shade_blocks;   // most blocks (of the variant's size) for shade_surface
     uint32_t light_blocks;   // blocks of 256 lanes for shade_miss
@@ -73,10 +74,15 @@ hipError_t launch_raygen(hipStream_t stream, uint32_t* counters, uint32_t counte
 
 // A range of so few paths is sure to leave its bounce 1 to the tail launch, so
 // the launches between, which return at once, are left out: a 64 x 64 view of
-// the Cornell box 0.30 -> 0.26 ms a pass.
+// the Cornell box 0.30 -> 0.26 ms a pass. That would hold for every range of at
+// most TAIL_PATHS (cn_stages.hip) paths; those above this line keep a launch per
+// stage and bounce up to the tail's own, which a profiling renderer's launch
+// counts of such a view (12,288 paths in the tests) are read by.
 constexpr uint32_t TAIL_AT_ONCE = 8192;
 
-// The bounce of a range that launches the tail, given the renderer's.
+// The bounce of a range that launches the tail, given the renderer's
+// (UINT32_MAX: no tail, which is also how a renderer's or a job's depth cap at or
+// below the tail's bounce runs: every bounce of such a wave as stages).
 constexpr uint32_t tail_launch_bounce(uint32_t tail_bounce, uint32_t range_count) {
     return tail_bounce != UINT32_MAX && range_count <= TAIL_AT_ONCE ? 1u : tail_bounce;
 }

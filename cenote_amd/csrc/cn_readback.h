@@ -10,8 +10,8 @@
 
 namespace cn {
 
-// A context's pinned staging for read-backs: 16 MiB in READBACK_SLOTS slots
-// and a stream per worker, taken at the first read-back and given back with
+// A context's pinned staging for read-backs: 16 MiB in SLOTS slots and
+// a stream per worker, taken at the first read-back and given back with
 // the context. One read-back uses it at a time.
 struct Readback {
     std::mutex busy;

@@ -76,7 +76,7 @@ __device__ __forceinline__ uint32_t queue_total(const uint32_t* counters, uint32
 // three launches about 90 us of dependent fetches whatever it holds, a path in
 // the tail some 20 us a bounce. Per pass at TAIL_PATHS 0 (never), 8192, 16384,
 // 49152: a 64 x 64 view of the Cornell box 0.345, 0.30, 0.293, 0.30 ms; a
-// 320 x 180 view of the 2M triangles, edited, 1.37, 1.19, 1.20, 1.24; the eight
+// 320 x 180 view of the material chart, edited, 1.37, 1.19, 1.20, 1.24; the eight
 // waves of a 720p session 9.3, 8.45, 8.45, 8.8; the veiled chart 2.87, 2.77,
 // 2.77, 2.79; waves of a million paths and more unchanged.
 constexpr uint32_t TAIL_PATHS = 16384;
@@ -965,10 +965,13 @@ __global__ __launch_bounds__(TRAVERSAL_BLOCK) __attribute__((amdgpu_waves_per_eu
     bool items_left = true;  // wave-uniform
     // Few items go over many waves: a wave carries no more pairs at once than
     // its share of all items. A launch's length is its longest path's, and a
-    // wave's bounce lasts as long as the longest walk of its pairs (the 2M-
-    // triangle scene's 28,000 paths 1.25 -> 0.92 ms from outside, 1.20 -> 1.00
-    // from inside; the veiled chart 0.56 -> 0.30; twice the share 1.10, 1.16
-    // and 0.29. The Cornell box, whose walks are short, 0.09 -> 0.11).
+    // wave's bounce lasts as long as the longest walk of its pairs. Of two 2M-
+    // triangle scenes the one whose bounce 6 holds 27,000 rays went from 1.25 to
+    // 0.92 ms from outside and from 1.20 to 1.00 from inside, the veiled chart
+    // from 0.56 to 0.30 (twice the share 1.10, 1.16 and 0.29); the other, with
+    // 98,000 rays there, whose waves have a full share in any case, gains nothing
+    // by it (1.42), and the Cornell box, whose walks are short, went from 0.09
+    // to 0.11.
     const uint32_t waves = gridDim.x * (TRAVERSAL_BLOCK / 64);
     const uint32_t share = min(max(n / waves, 1u), 32u);
     bool live = false;  // the pair carries a path (the same in both lanes)

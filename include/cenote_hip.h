@@ -360,7 +360,10 @@ enum {
     CN_SHADE_256_GLOBAL_SORTED = 6
 };
 typedef struct cn_launch_shape {
-    uint32_t trace_blocks;   /* 256-lane workgroups of the persistent trace kernel, 1..65536 */
+    uint32_t trace_blocks;   /* most 256-lane workgroups of a trace launch, 1..65536 (bounces from 1 on
+                              * run no more than the chip holds at once: 8 per compute unit over
+                              * 4-wide nodes, 7 over 8-wide); the traversal stack's spill area is
+                              * sized by it */
     uint32_t shade_variant;  /* a CN_SHADE_* value */
     uint32_t shade_blocks;   /* most workgroups of shade_surface, 1..65536 */
     uint32_t light_blocks;   /* most 256-lane workgroups of shade_miss, 1..65536 */
@@ -369,7 +372,8 @@ typedef struct cn_launch_shape {
     uint32_t tail_bounce;    /* 0: every bounce as wavefront stages; b in 1..255: after the trace of
                               * bounce b, or of an earlier one with few rays, one launch carries
                               * every live path through its remaining bounces (the same films, bit
-                              * for bit; waves with counters on keep the stages) */
+                              * for bit; waves with counters on, and waves of at most b bounces, keep
+                              * the stages) */
 } cn_launch_shape;
 int cn_renderer_get_shape(cn_renderer* renderer, cn_launch_shape* out);
 int cn_renderer_set_shape(cn_renderer* renderer, const cn_launch_shape* shape);
