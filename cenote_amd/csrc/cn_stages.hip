@@ -270,7 +270,8 @@ __global__ __launch_bounds__(BLOCK) void k_shade_miss(SceneView s, PathPool p, W
 // what the deep, sparse bounces need.
 
 // The 8-wide walk holds eight keys and refs through its sorting network:
-// at eight waves per SIMD (64 VGPRs) it spills, so it runs at fewer.
+// at eight waves per SIMD (64 VGPRs) it spills much of that, so it runs at
+// fewer (72 VGPRs, six spilled; the 4-wide kernel spills four of its 64).
 #ifndef TRACE8_WAVES
 #define TRACE8_WAVES 7
 #endif
