@@ -23,17 +23,18 @@
 
 namespace cn {
 
-hipError_t Readback::prepare() {
-    if (!slots) {
-        const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&slots), SLOT * SLOTS, hipHostMallocDefault);
-        if (e != hipSuccess) {
-            slots = nullptr;
-            return e;
+hipError_t Readback::prepare(int pairs, int workers) {
+    for (int w = 0; w < pairs; ++w)
+        if (!slots[w]) {
+            const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&slots[w]), 2 * SLOT, hipHostMallocDefault);
+            if (e != hipSuccess) {
+                slots[w] = nullptr;
+                return e;
+            }
         }
-    }
-    for (hipStream_t& s : streams)
-        if (!s) {
-            const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    for (int w = 0; w < workers; ++w)
+        if (!streams[w]) {
+            const hipError_t e = hipStreamCreateWithFlags(&streams[w], hipStreamNonBlocking);
             if (e != hipSuccess) return e;
         }
     return hipSuccess;
@@ -42,7 +43,8 @@ hipError_t Readback::prepare() {
 Readback::~Readback() {
     for (hipStream_t s : streams)
         if (s) (void)hipStreamDestroy(s);
-    if (slots) (void)hipHostFree(slots);
+    for (char* p : slots)
+        if (p) (void)hipHostFree(p);
 }
 
 namespace {
@@ -106,9 +108,13 @@ static int read_pieces(int device, Readback& rb, const ReadArray* arrays, int n)
             pieces.push_back({&a, first, std::min(step, a.count - first)});
     }
     if (pieces.empty()) return CN_OK;
+    const bool one = pieces.size() <= 4;  // copied by one stream, each piece into a slot of its own
+    const int workers = one ? 1 : int(std::min<size_t>(Readback::WORKERS, pieces.size() / 2));
     std::lock_guard<std::mutex> lock(rb.busy);
-    if (rb.prepare() != hipSuccess) {
-        // No pinned memory (or streams) to be had.
+    const bool first = !rb.used;
+    rb.used = true;
+    if ((one && first) || rb.prepare(one ? int(pieces.size() + 1) / 2 : workers, workers) != hipSuccess) {
+        // A context's first small read-back, or no pinned memory (or streams) to be had.
         (void)hipGetLastError();
         const ReadArray* last = nullptr;
         for (const Piece& p : pieces) {
@@ -119,11 +125,11 @@ static int read_pieces(int device, Readback& rb, const ReadArray* arrays, int n)
         return CN_OK;
     }
     auto copy = [&](int worker, int slot, const Piece& p) {
-        return hipMemcpyAsync(rb.slots + Readback::SLOT * slot, p.a->src + p.first, p.count * sizeof(float),
+        return hipMemcpyAsync(rb.slot(slot), p.a->src + p.first, p.count * sizeof(float),
                               hipMemcpyDeviceToHost, rb.streams[worker]);
     };
-    auto staged = [&](int slot) { return reinterpret_cast<const float*>(rb.slots + Readback::SLOT * slot); };
-    if (pieces.size() <= 4) {
+    auto staged = [&](int slot) { return reinterpret_cast<const float*>(rb.slot(slot)); };
+    if (one) {
         hipError_t e = hipSuccess;
         for (size_t k = 0; k < pieces.size() && e == hipSuccess; ++k) e = copy(0, int(k), pieces[k]);
         const hipError_t done = hipStreamSynchronize(rb.streams[0]);  // also before the slots are let go
@@ -156,7 +162,6 @@ static int read_pieces(int device, Readback& rb, const ReadArray* arrays, int n)
     // The calling thread is worker 0; a thread that cannot be had (the system's
     // limit, or no memory for its state) leaves its share to the others. Nothing
     // may leave this scope before they are joined.
-    const int workers = int(std::min<size_t>(Readback::WORKERS, pieces.size() / 2));
     std::vector<std::thread> threads;
     threads.reserve(workers);
     for (int w = 1; w < workers; ++w) {

@@ -10,17 +10,24 @@
 
 namespace cn {
 
-// A context's pinned staging for read-backs: 16 MiB in SLOTS slots and
-// a stream per worker, taken at the first read-back and given back with
-// the context. One read-back uses it at a time.
+// A context's pinned staging for read-backs: two 1 MiB slots and a stream per
+// worker, each taken by the first read-back that needs it and given back with
+// the context. The first read-back of a context, if it is one worker's, goes
+// without: making one worker's share takes 3 ms and all of it 8, which a
+// program that reads one small image back would not see again (that call 14 ms
+// with all of the staging made for it, 5 to 7 without, and 8 with a worker's;
+// later calls of 16 x 16 to 256 x 256 pixels are up to 45 us faster staged).
+// One read-back uses it at a time.
 struct Readback {
     std::mutex busy;
-    char* slots = nullptr;
+    bool used = false;
     static constexpr size_t SLOT = size_t(1) << 20;
     static constexpr int WORKERS = 8;
-    static constexpr int SLOTS = 2 * WORKERS;
+    char* slots[WORKERS] = {};  // two each
     hipStream_t streams[WORKERS] = {};
-    hipError_t prepare();
+    // Makes the first `pairs` workers' slots and the first `workers` ones' streams.
+    hipError_t prepare(int pairs, int workers);
+    char* slot(int i) const { return slots[i / 2] + SLOT * (i % 2); }
     ~Readback();
 };
 

@@ -19,6 +19,7 @@ thread_local long allocations_left = -1;  // -1: none fails
 std::atomic<long> copies_left{-1};
 std::atomic<int> in_flight{0};
 bool pinned = true;
+long pinned_bytes = 0, streams = 0;
 
 bool spend(std::atomic<long>& left) { return left.load() >= 0 && left.fetch_sub(1) == 0; }
 }  // namespace
@@ -37,6 +38,7 @@ hipError_t hipGetLastError(void) { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "made to fail"; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned int) {
     *p = pinned ? std::malloc(n) : nullptr;
+    pinned_bytes += n;
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 hipError_t hipHostFree(void* p) {
@@ -46,6 +48,7 @@ hipError_t hipHostFree(void* p) {
 hipError_t hipFree(void*) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned int) {
     *s = reinterpret_cast<hipStream_t>(std::malloc(1));
+    ++streams;
     return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t s) {
@@ -101,6 +104,12 @@ int main() {
     constexpr size_t SLOT = cn::Readback::SLOT / sizeof(float);
     cn::Readback rb;
     Call call;
+    // A context's first small image takes no staging, the next ones what one
+    // worker needs, and a large one the rest.
+    check(call.run(rb, 1000, 3.0f) == CN_OK && call.whole(3.0f) && pinned_bytes == 0 && streams == 0, "first", 1000);
+    check(call.run(rb, 1000, 3.0f) == CN_OK && call.whole(3.0f) && pinned_bytes <= 2 << 20 && streams == 1, "next", 1000);
+    check(call.run(rb, 4 * SLOT, 3.0f) == CN_OK && pinned_bytes <= 4 << 20 && streams == 1, "next", 4 * SLOT);
+    check(call.run(rb, 40 * SLOT, 3.0f) == CN_OK && pinned_bytes <= 16 << 20 && streams == 8, "next", 40 * SLOT);
     // One piece, several in one copy each, several workers, all of them; last pieces not full.
     for (size_t count : {size_t(1), SLOT, SLOT + 1, 4 * SLOT, 4 * SLOT + 1, 9 * SLOT + 7, 40 * SLOT + 3})
         for (float divisor : {1.0f, 3.0f})
