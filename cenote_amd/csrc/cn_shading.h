@@ -109,10 +109,18 @@ __device__ __forceinline__ float tab3(const float* t, uint32_t off, float x, flo
     return lerpf(tab2(t, off + 256u * i, 16, 16, x, y), tab2(t, off + 256u * j, 16, 16, x, y), fz - float(i));
 }
 
-// An index of refraction comes from the scene, at any scale (cn_math.h): the
-// quotients of one are the operators' wherever it is not the closure's own
-// (0, 2^-25 to 2^25, or infinite).
-__device__ __forceinline__ float ior_remap(float eta) { return sqrt_n(fabsf(eta - 1.0f) / (eta + 1.0f)); }
+// An index of refraction comes from the scene, at any scale (cn_math.h): with
+// SCENE_IOR the quotients are the operators', without it div_n's, for the
+// closure's own index (0, 2^-25 to 2^25, or infinite).
+template <bool SCENE_IOR>
+__device__ __forceinline__ float ior_quotient(float a, float b) {
+    return SCENE_IOR ? a / b : div_n(a, b);
+}
+
+template <bool SCENE_IOR = false>
+__device__ __forceinline__ float ior_remap(float eta) {
+    return sqrt_n(ior_quotient<SCENE_IOR>(fabsf(eta - 1.0f), eta + 1.0f));
+}
 
 // --- EON diffuse (openpbr.slang:134-175) ----------------------------------------
 
@@ -176,24 +184,24 @@ __device__ __forceinline__ v3 fresnel_schlick(v3 f0, float cosine) {
     return f0 + (((1.0f - f0) * m2) * m2) * m;
 }
 
-template <bool SCENE_IOR = false>  // not the closure's own
+template <bool SCENE_IOR = false>
 __device__ __forceinline__ float fresnel_dielectric(float eta, float cosine) {
-    const auto quotient = [](float a, float b) { return SCENE_IOR ? a / b : div_n(a, b); };
     const float mu = fabsf(cosine);
     const float sin2 = 1.0f - mu * mu;
-    const float cos2t = 1.0f - quotient(sin2, eta * eta);
+    const float cos2t = 1.0f - ior_quotient<SCENE_IOR>(sin2, eta * eta);
     if (cos2t < 0.0f) return 1.0f;
     const float t0 = sqrt_n(cos2t);
     const float t1 = eta * t0;
     const float t2 = eta * mu;
-    const float rs = quotient(mu - t1, mu + t1);
-    const float rp = quotient(t0 - t2, t0 + t2);
+    const float rs = ior_quotient<SCENE_IOR>(mu - t1, mu + t1);
+    const float rp = ior_quotient<SCENE_IOR>(t0 - t2, t0 + t2);
     return (rs * rs + rp * rp) / 2.0f;
 }
 
+template <bool SCENE_IOR = false>
 __device__ __forceinline__ float fresnel_dielectric_avg(float eta) {
     if (eta < 1.0f) return 0.997118f + eta * (0.1014f - eta * (0.965241f + eta * 0.130607f));
-    return (eta - 1.0f) / (4.08567f + 1.00071f * eta);
+    return ior_quotient<SCENE_IOR>(eta - 1.0f, 4.08567f + 1.00071f * eta);
 }
 
 __device__ __forceinline__ v3 fresnel_ms(v3 fss, float eAvg) {
@@ -230,12 +238,12 @@ __device__ __forceinline__ v3 reflection_scale(const float* t, float rough, floa
 template <bool SCENE_IOR = false>
 __device__ __forceinline__ float dielectric_albedo(const float* t, float rough, float mu, float eta) {
     if (eta < 1.0f) return fresnel_dielectric<SCENE_IOR>(eta, mu);
-    return tab3(t, T_DIELECTRIC_E, rough, mu, ior_remap(eta));
+    return tab3(t, T_DIELECTRIC_E, rough, mu, ior_remap<SCENE_IOR>(eta));
 }
 
 // openpbr.slang:371-384
 __device__ __forceinline__ v3 coat_darkening(const Mat& m, float rough, float mu, float baseFresnel) {
-    const float fssCoat = fresnel_dielectric_avg(m.coatIor);
+    const float fssCoat = fresnel_dielectric_avg<true>(m.coatIor);
     const float kRough = 1.0f - (1.0f - fssCoat) / (m.coatIor * m.coatIor);
     const float kSmooth = fresnel_dielectric<true>(m.coatIor, mu);
     const float roughDiffuse = lerpf(1.0f, rough, saturate(m.specularWeight * baseFresnel));
@@ -298,7 +306,7 @@ __device__ inline Closure resolve_closure(const float* t, const Mat& m, v3 wo, b
     v3 coatAtten = S3(1.0f);
     if (coated) {
         c.coatE = dielectric_albedo<true>(t, coatRough, mu, m.coatIor);
-        const float fssCoat = fresnel_dielectric_avg(m.coatIor);
+        const float fssCoat = fresnel_dielectric_avg<true>(m.coatIor);
         c.coatScale = reflection_scale(t, coatRough, mu, S3(fssCoat)).x;
         coatAtten = vlerp(S3(1.0f), m.coatColor * (1.0f - c.coatE), m.coatWeight) * coat_darkening(m, rough, mu, f0);
     }
