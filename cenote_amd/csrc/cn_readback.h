@@ -32,8 +32,8 @@ struct Readback {
 };
 
 // One array to read back: `count` f32 from device memory `src`, each divided
-// by `divisor` where that is not 1; with `width`, the values are `lanes`-wide
-// pixels in band order (band_pixel) and land row-major.
+// by `divisor` where that is not 1; with `width`, the values are pixels of
+// `lanes` (4 or 1) values in band order (band_pixel) and land row-major.
 struct ReadArray {
     const float* src;
     float* dst;  // null: skipped
